@@ -68,6 +68,9 @@ SIGNATURES: dict[str, list] = {
     "fd_rope": [_p, _p, _p, _p, _i, _rows, _rows, _rows, _rows, _i, _p],
     "fd_linear": [_p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _i, _i, _p],
     "fd_linear_fp8": [_p, _p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _i, _p],
+    "fd_linear_fp8_wide": [_p, _p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _p, _l, _i, _p],
+    "fd_linear_fp8_wide_scratch": [_l, _l, _l, ctypes.POINTER(_l)],
+    "fd_gate_up_fp8_wide": [_p, _p, _p, _p, _l, _l, _l, _l, _i, _p],
     "fd_post_attn_mlp_fp8": [_p, _p, _p, _p, _i, _p, _p, _p, _p, _l, _l, _l, _f, _i, _p],
     "fd_linear_tiled": [_p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l,
                         ctypes.POINTER(FdTile), _i, _i, _p],

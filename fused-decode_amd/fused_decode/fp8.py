@@ -12,17 +12,19 @@ activations, so the only approximation is the weight quantisation itself:
 
     y[m, n] = round(scale[n] * sum_k e4m3(q[n, k]) * x[m, k] + bias[n] + row_add[m, n])
 
-A decode GEMV at M <= 16 streams one byte per weight instead of two. There is no
-reference counterpart (the reference has fp16/bf16 weights only); this is the
+A decode GEMV at M <= 16 streams one byte per weight instead of two; above 16
+rows a tiled GEMM does, with the same arithmetic. There is no reference counterpart (the reference has fp16/bf16 weights only); this is the
 low-precision weight format its roadmap leaves for last.
 """
 
 from __future__ import annotations
 
+import ctypes
 import math
 import warnings
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._checks import check
@@ -44,6 +46,27 @@ def _slow_path(why: str) -> None:
         warnings.warn(f"linear_decode_fp8: {why}; computing a float32 product of the decoded weights "
                       "(same values, about 4x the weight traffic of the fp8 kernels)", RuntimeWarning,
                       stacklevel=5)  # _slow_path, the plan's helper, the plan, linear_decode_fp8, its caller
+
+
+def _only_values(*tensors) -> bool:
+    """Whether these are plain tensors that nothing records or transforms, so that a
+    launch on their pointers says all that the torch formula would: no gradient
+    wanted, no forward-mode level, no vmap or tracing."""
+    if forward_ad._current_level >= 0 or torch.compiler.is_compiling():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)
+                              or torch._C._functorch.is_functorch_wrapped_tensor(t)):
+            return False
+    return True
+
+
+def _wide_scratch(m: int, n: int, k: int) -> int:
+    """Bytes of scratch fd_linear_fp8_wide's preferred K split takes."""
+    out = ctypes.c_int64(0)
+    _lib.check("fd_linear_fp8_wide_scratch", _lib.lib().fd_linear_fp8_wide_scratch(m, n, k, ctypes.byref(out)))
+    return out.value
 
 
 def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
@@ -78,10 +101,10 @@ def linear_decode_fp8(
 ) -> torch.Tensor:
     """``y = (x @ dequantize(weight, scale).T) (+ bias) (+ row_add)`` with E4M3
     ``weight [N, K]`` and float32 ``scale [N]``; argument rules as
-    ``linear_decode`` (ops.py:212-280 of the reference). Up to 16 rows with
-    ``K % 16 == 0`` this is the HIP fp8 GEMV; other shapes compute a float32
-    product of the decoded weights (same values, several times the traffic: a
-    RuntimeWarning says so once per reason)."""
+    ``linear_decode`` (ops.py:212-280 of the reference). With ``K % 16 == 0`` this is
+    the HIP fp8 GEMV up to 16 rows and a tiled GEMM above; other shapes compute a
+    float32 product of the decoded weights (same values, several times the
+    traffic: a RuntimeWarning says so once per reason)."""
     try:
         key = ("linear_fp8", _sig(x), _sig(weight), _sig(scale), _sig(bias), _sig(row_add), _sig(out))
         plan = _PLANS.get(key)
@@ -120,13 +143,16 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
     x2p = x.reshape(m, k)
     x_copy = x2p.stride(1) != 1  # gathered per call into contiguous rows
     why = None
-    if m > _HAND_LIMIT:
-        why = f"{m} rows is above the kernels' {_HAND_LIMIT}"
+    if k == 0:
+        why = "K is 0" if m > _HAND_LIMIT else None
     elif not (weight.stride(1) == 1 and (n == 1 or weight.stride(0) % 16 == 0) and k % 16 == 0):
         why = "the codes are not 16-byte rows with K % 16 == 0"
     elif not x_copy and m > 1 and x2p.stride(0) % 8 != 0:
         why = "x rows are not 16-byte aligned with unit stride"
     if why is not None:
+        if m > _HAND_LIMIT:
+            why = f"{m} rows is above the decode kernels' {_HAND_LIMIT} and {why}"
+
         def fallback(x, w, sc, b, r, o):
             x2 = x.reshape(m, k)
             return slow(x2.contiguous() if x_copy else x2, w, sc, b, r, alloc(x) if o is None else o, why)
@@ -140,6 +166,9 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
     dense_sc = _dense(scale)
     sxm = k if x_copy else int(x2p.stride(0))
     call = native().linear_fp8
+    wide = m > _HAND_LIMIT
+    if wide:
+        call_wide, scratch_bytes = native().linear_fp8_wide, _wide_scratch(m, n, k)
 
     def run(x, w, sc, b, r, o):
         y = alloc(x) if o is None else o
@@ -150,8 +179,20 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
             return slow(x2, w, sc, b, r, y, "the codes are not 16-byte rows with K % 16 == 0")
         if x2.data_ptr() % 16:
             return slow(x2, w, sc, b, r, y, "x rows are not 16-byte aligned with unit stride")
+        if wide and not _only_values(x, sc, b, r):
+            return slow(x2, w, sc, b, r, y, "a gradient or a transform is asked for")
         if r is not None and r_flat:  # indexed in place through (srm, srn), or copied when its dims do not merge
             r = r.expand(expected).reshape(m, n)
+        if wide:
+            part = x2.new_empty(scratch_bytes // 4, dtype=torch.float32) if scratch_bytes else None
+            status = call_wide(y.data_ptr(), x2.data_ptr(), w.data_ptr(),
+                               (sc if dense_sc else sc.contiguous()).data_ptr(), None if b is None else b.data_ptr(),
+                               bcode, None if r is None else r.data_ptr(), rcode, m, n, k, sxm, int(w.stride(0)), sb,
+                               srm, srn, n, 1, None if part is None else part.data_ptr(), scratch_bytes, act,
+                               _raw_stream(dev))
+            if status:
+                fail("fd_linear_fp8_wide", status)
+            return y
         status = call(y.data_ptr(), x2.data_ptr(), w.data_ptr(), (sc if dense_sc else sc.contiguous()).data_ptr(),
                       None if b is None else b.data_ptr(), bcode, None if r is None else r.data_ptr(), rcode,
                       m, n, k, sxm, int(w.stride(0)), sb, srm, srn, n, 1, act, _raw_stream(dev))
@@ -173,8 +214,9 @@ def post_attn_mlp_fp8(
     """``post_attn_mlp`` with E4M3 weights (``w_gate_up [2I, H]``, ``w_down [H, I]``)
     and their float32 per-row scales: the same four rounding points (reference
     reference.py:66-79), each projection as ``linear_decode_fp8``. Two HIP launches
-    up to 16 rows (from 5 the MFMA gate/up normalises inside its kernel);
-    otherwise composed from the operators."""
+    up to 16 rows (from 5 the MFMA gate/up normalises inside its kernel); above,
+    the norm, one gate/up + SwiGLU launch and the down product; otherwise composed
+    from the operators."""
     try:
         key = ("mlp_fp8", _sig(hidden), _sig(norm_weight), _sig(w_gate_up), _sig(gate_up_scale), _sig(w_down),
                _sig(down_scale), eps)
@@ -199,11 +241,27 @@ def _plan_mlp_fp8(hidden, norm_weight, w_gate_up, gate_up_scale, w_down, down_sc
         gate, up = linear_decode_fp8(normed, wgu, sgu).split(i, dim=-1)
         return linear_decode_fp8(swiglu(gate, up), wd, sd, row_add=x)
 
-    if not (0 < m <= _HAND_LIMIT and w_gate_up.is_contiguous() and w_down.is_contiguous()
-            and h % 16 == 0 and i % 16 == 0):
+    if not (m > 0 and w_gate_up.is_contiguous() and w_down.is_contiguous() and h % 16 == 0
+            and i % 16 == 0) or (m > _HAND_LIMIT and i == 0):
         return composed
     shape = tuple(hidden.shape)
     dense_h, dense_nw, dense_s = _dense(hidden), _dense(norm_weight), _dense(gate_up_scale) and _dense(down_scale)
+    if m > _HAND_LIMIT:
+        gate_up, act_w, dev_w = native().gate_up_fp8_wide, DTYPE_CODE[hidden.dtype], hidden.device.index
+        mid_shape = (*shape[:-1], i)
+
+        def wide(x, nw, wgu, sgu, wd, sd):
+            normed = rms_norm(x, nw, eps=eps)
+            if wgu.data_ptr() % 16 or not _only_values(normed, sgu):
+                gate, up = linear_decode_fp8(normed, wgu, sgu).split(i, dim=-1)
+                return linear_decode_fp8(swiglu(gate, up), wd, sd, row_add=x)
+            mid = normed.new_empty(mid_shape)
+            status = gate_up(mid.data_ptr(), normed.data_ptr(), wgu.data_ptr(),
+                             (sgu if dense_s else sgu.contiguous()).data_ptr(), m, h, i, h, act_w, _raw_stream(dev_w))
+            if status:
+                fail("fd_gate_up_fp8_wide", status)
+            return linear_decode_fp8(mid, wd, sd, row_add=x)
+        return wide
     call, act, nwc, dev = (native().post_attn_mlp_fp8, DTYPE_CODE[hidden.dtype], DTYPE_CODE[norm_weight.dtype],
                            hidden.device.index)
 

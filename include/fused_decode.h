@@ -262,6 +262,36 @@ int fd_linear_fp8(void* y, const void* x, const void* w8, const float* w_scale,
                   void* stream);
 
 /*
+ * fd_linear_fp8's product for any number of rows (meant for M > 16): a tiled
+ * MFMA GEMM with the codes decoded exactly and float32 sums. K > 0. Where the
+ * output has fewer tiles than the GPU has CUs, K is split over workgroups whose
+ * float32 sums go through `scratch` (16-byte aligned, caller-owned, not shared
+ * with a call that may overlap); fd_linear_fp8_wide_scratch gives the bytes that
+ * the preferred split needs (0: none). A smaller `scratch_bytes` lowers the
+ * split, down to none with scratch NULL. The sums are added in a fixed order.
+ * K % 16 == 0 and 16-byte aligned rows (else FD_EUNSUPPORTED). No reference
+ * counterpart (see fd_linear_fp8).
+ */
+int fd_linear_fp8_wide(void* y, const void* x, const void* w8, const float* w_scale,
+                       const void* bias, int bias_dtype, const void* row_add, int row_dtype,
+                       int64_t M, int64_t N, int64_t K, int64_t sxm, int64_t swn, int64_t sb,
+                       int64_t srm, int64_t srn, int64_t sym, int64_t syn, float* scratch,
+                       int64_t scratch_bytes, int act_dtype, void* stream);
+int fd_linear_fp8_wide_scratch(int64_t M, int64_t N, int64_t K, int64_t* bytes);
+
+/*
+ * The gate/up half of an MLP with FP8 weights for any number of rows (meant for
+ * M > 16): mid[m,j] = round(silu(round(g)) * round(u)) with g and u the products
+ * of x [M,H] (row stride sxm, already normalised) with rows j and I + j of
+ * w_gate_up8 [2I,H] (contiguous), as fd_linear_fp8 computes them. mid is [M,I]
+ * contiguous. H % 16 == 0 and 16-byte aligned rows (else FD_EUNSUPPORTED). No
+ * reference counterpart.
+ */
+int fd_gate_up_fp8_wide(void* mid, const void* x, const void* w_gate_up8,
+                        const float* gate_up_scale, int64_t M, int64_t H, int64_t I, int64_t sxm,
+                        int act_dtype, void* stream);
+
+/*
  * fd_post_attn_mlp with FP8 weights: w_gate_up8 [2I,H] and w_down8 [H,I] E4M3
  * codes (contiguous) with per-row float32 scales gate_up_scale [2I] and
  * down_scale [H]; each projection is fd_linear_fp8's product, with the same four

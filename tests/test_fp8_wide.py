@@ -1,0 +1,39 @@
+"""Argument checks of the wide E4M3 entry points (before any HIP call)."""
+
+from __future__ import annotations
+
+import ctypes
+
+FAKE = 0x1000
+
+
+def test_wide_entry_points_reject():
+    from fused_decode import _lib as L
+
+    lib = L.lib()
+
+    def lin(m=32, n=64, k=128, sxm=128, swn=128, x=FAKE, w=FAKE, bias=None, bias_dtype=0, act=0):
+        return lib.fd_linear_fp8_wide(FAKE, x, w, FAKE, bias, bias_dtype, None, 0, m, n, k, sxm, swn, 0, 0, 0, n, 1,
+                                      None, 0, act, None)
+
+    assert lin(act=2) == L.FD_EINVAL and lin(k=0) == L.FD_EINVAL and lin(m=-1) == L.FD_EINVAL
+    assert lin(sxm=-8) == L.FD_EINVAL and lin(x=None) == L.FD_EINVAL and lin(bias=FAKE, bias_dtype=1) == L.FD_EINVAL
+    assert lin(k=120) == L.FD_EUNSUPPORTED and lin(sxm=132) == L.FD_EUNSUPPORTED
+    assert lin(swn=136) == L.FD_EUNSUPPORTED and lin(w=FAKE + 8) == L.FD_EUNSUPPORTED
+    assert lin(m=0) == L.FD_OK and lin(n=0) == L.FD_OK
+    gate = lambda m=32, h=128, i=64, x=FAKE, act=0: lib.fd_gate_up_fp8_wide(FAKE, x, FAKE, FAKE, m, h, i, h, act, None)
+    assert gate(act=5) == L.FD_EINVAL and gate(h=0) == L.FD_EINVAL and gate(i=0) == L.FD_EINVAL
+    assert gate(x=None) == L.FD_EINVAL and gate(h=120) == L.FD_EUNSUPPORTED and gate(m=0) == L.FD_OK
+
+
+def test_wide_scratch_follows_the_tiles():
+    """No split, so no scratch, once the output tiles cover the GPU; else float32 sums for each split."""
+    from fused_decode import _lib as L
+
+    out = ctypes.c_int64(-1)
+    ask = lambda m, n, k: (L.lib().fd_linear_fp8_wide_scratch(m, n, k, ctypes.byref(out)), out.value)
+    assert ask(0, 64, 64) == (L.FD_OK, 0) and ask(32, 128, 256) == (L.FD_OK, 0)
+    assert ask(300, 28672, 4096) == (L.FD_OK, 0)
+    rc, got = ask(100, 4096, 14336)
+    assert rc == L.FD_OK and got > 0 and got % (100 * 4096 * 4) == 0
+    assert L.lib().fd_linear_fp8_wide_scratch(-1, 1, 1, ctypes.byref(out)) == L.FD_EINVAL
