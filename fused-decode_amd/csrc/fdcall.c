@@ -102,6 +102,9 @@ static int (*p_pre_attn_qkv)(void*, void*, const void*, const void*, int, const 
 static int (*p_linear_fp8)(void*, const void*, const void*, const float*, const void*, int,
                            const void*, int, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,
                            int64_t, int64_t, int64_t, int64_t, int, void*);
+static int (*p_linear_kn)(void*, const void*, const void*, const void*, int, const void*, int,
+                          int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,
+                          int64_t, int64_t, int64_t, float*, int64_t, int, void*);
 static int (*p_linear_fp8_wide)(void*, const void*, const void*, const float*, const void*, int,
                                 const void*, int, int64_t, int64_t, int64_t, int64_t, int64_t,
                                 int64_t, int64_t, int64_t, int64_t, int64_t, float*, int64_t, int,
@@ -162,6 +165,10 @@ WRAP(linear_fp8, "pppppipillllllllllis",
      p_linear_fp8(a[0].p, a[1].p, a[2].p, (const float*)a[3].p, a[4].p, a[5].i, a[6].p, a[7].i,
                   a[8].l, a[9].l, a[10].l, a[11].l, a[12].l, a[13].l, a[14].l, a[15].l, a[16].l,
                   a[17].l, a[18].i, a[19].p))
+WRAP(linear_kn, "ppppipilllllllllllplis",
+     p_linear_kn(a[0].p, a[1].p, a[2].p, a[3].p, a[4].i, a[5].p, a[6].i, a[7].l, a[8].l, a[9].l,
+                 a[10].l, a[11].l, a[12].l, a[13].l, a[14].l, a[15].l, a[16].l, a[17].l,
+                 (float*)a[18].p, a[19].l, a[20].i, a[21].p))
 WRAP(linear_fp8_wide, "pppppipillllllllllplis",
      p_linear_fp8_wide(a[0].p, a[1].p, a[2].p, (const float*)a[3].p, a[4].p, a[5].i, a[6].p, a[7].i,
                        a[8].l, a[9].l, a[10].l, a[11].l, a[12].l, a[13].l, a[14].l, a[15].l,
@@ -225,6 +232,7 @@ static PyObject* w_bind(PyObject* self, PyObject* arg) {
   RESOLVE(p_post_attn_mlp, "fd_post_attn_mlp");
   RESOLVE(p_pre_attn_qkv, "fd_pre_attn_qkv");
   RESOLVE(p_linear_fp8, "fd_linear_fp8");
+  RESOLVE(p_linear_kn, "fd_linear_kn");
   RESOLVE(p_linear_fp8_wide, "fd_linear_fp8_wide");
   RESOLVE(p_gate_up_fp8_wide, "fd_gate_up_fp8_wide");
   RESOLVE(p_post_attn_mlp_fp8, "fd_post_attn_mlp_fp8");
@@ -250,6 +258,7 @@ static PyMethodDef methods[] = {
     FAST(post_attn_mlp),
     FAST(pre_attn_qkv),
     FAST(linear_fp8),
+    FAST(linear_kn),
     FAST(linear_fp8_wide),
     FAST(gate_up_fp8_wide),
     FAST(post_attn_mlp_fp8),

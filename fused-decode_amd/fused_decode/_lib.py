@@ -68,6 +68,8 @@ SIGNATURES: dict[str, list] = {
     "fd_rope": [_p, _p, _p, _p, _i, _rows, _rows, _rows, _rows, _i, _p],
     "fd_linear": [_p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _i, _i, _p],
     "fd_linear_fp8": [_p, _p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _i, _p],
+    "fd_linear_kn": [_p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _p, _l, _i, _p],
+    "fd_linear_kn_scratch": [_l, _l, _l, ctypes.POINTER(_l)],
     "fd_linear_fp8_wide": [_p, _p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _p, _l, _i, _p],
     "fd_linear_fp8_wide_scratch": [_l, _l, _l, ctypes.POINTER(_l)],
     "fd_gate_up_fp8_wide": [_p, _p, _p, _p, _l, _l, _l, _l, _i, _p],
@@ -176,6 +178,13 @@ def native():
 def fail(func: str, status: int) -> None:
     """Raise the library's error for a non-OK ``status`` of ``func``."""
     raise FusedDecodeError(func, status, native().last_error())
+
+
+def scratch_bytes(func: str, m: int, n: int, k: int) -> int:
+    """Bytes of scratch the preferred K split of an [M, N, K] product takes (``func``: a *_scratch entry point)."""
+    out = ctypes.c_int64(0)
+    check(func, getattr(lib(), func)(m, n, k, ctypes.byref(out)))
+    return out.value
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)

@@ -19,7 +19,6 @@ low-precision weight format its roadmap leaves for last.
 
 from __future__ import annotations
 
-import ctypes
 import math
 import warnings
 
@@ -60,13 +59,6 @@ def _only_values(*tensors) -> bool:
                               or torch._C._functorch.is_functorch_wrapped_tensor(t)):
             return False
     return True
-
-
-def _wide_scratch(m: int, n: int, k: int) -> int:
-    """Bytes of scratch fd_linear_fp8_wide's preferred K split takes."""
-    out = ctypes.c_int64(0)
-    _lib.check("fd_linear_fp8_wide_scratch", _lib.lib().fd_linear_fp8_wide_scratch(m, n, k, ctypes.byref(out)))
-    return out.value
 
 
 def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
@@ -168,7 +160,7 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
     call = native().linear_fp8
     wide = m > _HAND_LIMIT
     if wide:
-        call_wide, scratch_bytes = native().linear_fp8_wide, _wide_scratch(m, n, k)
+        call_wide, scratch_bytes = native().linear_fp8_wide, _lib.scratch_bytes("fd_linear_fp8_wide_scratch", m, n, k)
 
     def run(x, w, sc, b, r, o):
         y = alloc(x) if o is None else o

@@ -481,6 +481,11 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
     sb = int(bias.stride(0)) if bias is not None else 0
     rcode = DTYPE_CODE[row_add.dtype] if row_add is not None else act
     srm, srn, r_flat = ra if ra is not None else (0, 0, False)
+    # a weight stored [K, N] (a transposed view) has its own kernel; a forced tile
+    # names one of the [N, K] kernels, and is checked by them
+    kn = swn == 1 and swk != 1 and n % 8 == 0 and swk % 8 == 0 and k > 0 and not _env("FUSED_DECODE_LINEAR")
+    if kn:
+        call_kn, scratch_bytes = native().linear_kn, _lib.scratch_bytes("fd_linear_kn_scratch", m, n, k)
 
     def run(x, w, b, r, out):
         y = alloc(x) if out is None else out
@@ -488,6 +493,15 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
             x = x.reshape(m, k)
         if r_flat:
             r = r.expand(expected).reshape(m, n)
+        if kn:
+            part = x.new_empty(scratch_bytes // 4, dtype=torch.float32) if scratch_bytes else None
+            status = call_kn(y.data_ptr(), x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), bcode,
+                             None if r is None else r.data_ptr(), rcode, m, n, k, xr.row, xr.col, swk, sb, srm, srn, n,
+                             1, None if part is None else part.data_ptr(), scratch_bytes, act, _raw_stream(dev))
+            if status == 0:
+                return y
+            if status != FD_EUNSUPPORTED:  # unaligned weight rows: the kernel for any strides
+                fail("fd_linear_kn", status)
         status = call(y.data_ptr(), x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), bcode,
                       None if r is None else r.data_ptr(), rcode, m, n, k, xr.row, xr.col, swn, swk, sb, srm,
                       srn, n, 1, tile, kcode, act, _raw_stream(dev))

@@ -244,6 +244,22 @@ int fd_pre_attn_qkv(void* y, void* normed, const void* hidden, const void* norm_
                     float eps, int kind, int act_dtype, void* stream);
 
 /*
+ * fd_linear's product for a weight stored [K, N] (column n's elements swk apart,
+ * consecutive n adjacent), as a transposed view has it: y[m,n] = round(sum_k
+ * x[m,k] * w[k*swk + n] + bias[n] + row_add[m,n]). M <= 16, K > 0; any x strides.
+ * K is split over workgroups whose float32 sums go through `scratch`
+ * (caller-owned, not shared with a call that may overlap); fd_linear_kn_scratch
+ * gives the bytes of the preferred split (0: none). Less lowers the split, down
+ * to none with scratch NULL. The sums are added in a fixed order. N % 8 == 0 and
+ * 16-byte aligned rows of w (else FD_EUNSUPPORTED: fd_linear takes any strides).
+ */
+int fd_linear_kn(void* y, const void* x, const void* w, const void* bias, int bias_dtype,
+                 const void* row_add, int row_dtype, int64_t M, int64_t N, int64_t K, int64_t sxm,
+                 int64_t sxk, int64_t swk, int64_t sb, int64_t srm, int64_t srn, int64_t sym,
+                 int64_t syn, float* scratch, int64_t scratch_bytes, int act_dtype, void* stream);
+int fd_linear_kn_scratch(int64_t M, int64_t N, int64_t K, int64_t* bytes);
+
+/*
  * GEMV with FP8 weights (OCP E4M3, one byte per weight, row stride swn in bytes)
  * and one float32 scale per output row:
  *   y[m,n] = round(w_scale[n] * sum_k e4m3(w8[n,k]) * x[m,k] + bias[n] + row_add[m,n])

@@ -1,4 +1,4 @@
-"""Argument checks of the wide E4M3 entry points (before any HIP call)."""
+"""Argument checks of the entry points that take scratch (before any HIP call)."""
 
 from __future__ import annotations
 
@@ -37,3 +37,23 @@ def test_wide_scratch_follows_the_tiles():
     rc, got = ask(100, 4096, 14336)
     assert rc == L.FD_OK and got > 0 and got % (100 * 4096 * 4) == 0
     assert L.lib().fd_linear_fp8_wide_scratch(-1, 1, 1, ctypes.byref(out)) == L.FD_EINVAL
+
+
+def test_kn_entry_points_reject():
+    from fused_decode import _lib as L
+
+    lib = L.lib()
+
+    def lin(m=4, n=64, k=128, sxk=1, swk=64, x=FAKE, w=FAKE, bias=None, bias_dtype=0, act=0):
+        return lib.fd_linear_kn(FAKE, x, w, bias, bias_dtype, None, 0, m, n, k, k, sxk, swk, 0, 0, 0, n, 1, None, 0,
+                                act, None)
+
+    assert lin(act=2) == L.FD_EINVAL and lin(k=0) == L.FD_EINVAL and lin(m=17) == L.FD_EINVAL
+    assert lin(sxk=-1) == L.FD_EINVAL and lin(x=None) == L.FD_EINVAL and lin(bias=FAKE, bias_dtype=1) == L.FD_EINVAL
+    assert lin(n=60) == L.FD_EUNSUPPORTED and lin(swk=68) == L.FD_EUNSUPPORTED
+    assert lin(w=FAKE + 8) == L.FD_EUNSUPPORTED
+    assert lin(m=0) == L.FD_OK and lin(n=0) == L.FD_OK
+    out = ctypes.c_int64(-1)
+    assert lib.fd_linear_kn_scratch(4, 4096, 4096, ctypes.byref(out)) == L.FD_OK
+    assert out.value > 0 and out.value % (4 * 4096 * 4) == 0
+    assert lib.fd_linear_kn_scratch(4, 65536, 4096, ctypes.byref(out)) == L.FD_OK and out.value == 0
