@@ -5,7 +5,10 @@
 //   add_rms: s = x + r (float32); ro = round(s); y = round(s * rsqrt(mean(s^2) + eps) * w)
 // The norm always sees the float32 sum, never the rounded residual.
 //
-// Three kernels:
+// Four kernels:
+//   rms_rows_kernel - unit column stride, rows of any alignment and n >= 8: n <= 256
+//                     (several rows per wave) and what the next two don't take up
+//                     to n = 8192.
 //   rms_wave_kernel - unit column stride, n % 8 == 0, 16-byte aligned rows,
 //                     n <= 8192: one wave per row, the row in registers.
 //   rms_vec_kernel  - the same layouts for 8192 < n <= 16384: one 256-thread
@@ -15,6 +18,7 @@
 //                     pass re-reads through L2).
 // Reduction: wave64 shuffles, then one LDS exchange across the workgroup's waves.
 #include "fd_device.h"
+#include "fd_gemv.h"
 #include "fd_host.h"
 #include "fd_internal.h"
 
@@ -190,6 +194,128 @@ __global__ __launch_bounds__(256, !ADD && VPL <= 8 ? 8 : 1) void rms_wave_kernel
   }
 }
 
+// LPR lanes per row (a power of two; 64 / LPR rows per wave), VPL vectors of 8 per
+// lane, RPT rows per lane group, every row's loads issued before the first
+// reduction. Vectors are loaded and stored as 2-byte aligned 16-byte words, which
+// gfx950 does in one instruction at any address, so rows may start anywhere. Where
+// n % 8 != 0 the last vector lies at n - 8: its first elements, which the vector
+// before it holds too, are left out of the sum and written twice with one value
+// (every load of a row comes before its first store, so in place as well).
+//
+// Short rows are why LPR varies: with a wave per row an attention head's norm (n =
+// 128) uses 16 of 64 lanes and moves 512 bytes per wave before it ends. Of the 32
+// query heads of 2048 tokens (float16, views of a QKV buffer, float32 weight): n =
+// 64 / 80 / 128 / 256 13.8 / 14.5 / 15.1 / 17.2 us with a wave per row, 4.3 / 6.0 /
+// 7.0 / 12.5 here (n = 128: 4.8 TB/s), and one token's in 2.0 either way. Rows that are not
+// 16-byte aligned, which a workgroup per row reads twice in 2-byte loads: 2048 x 4097
+// 15.9 -> 8.8 us, 8192 x 1025 18.5 -> 9.7, 4096 x 8191 68.8 -> 27.0, 65536 x 100 42.0
+// -> 6.9, one row of 4097 6.1 -> 4.3. Aligned rows past 256 stay with the wave kernel,
+// whose weights sit in LDS (4096 x 8192 23.0 us).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <typename T>
+__device__ __forceinline__ typename Vec8<T>::type load8_any(const T* p) {
+  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+  return __builtin_bit_cast(typename Vec8<T>::type, v);
+}
+template <typename T>
+__device__ __forceinline__ void store8_any(T* p, typename Vec8<T>::type v) {
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4_any*>(p));
+}
+// 8 norm weights at any address, in their storage form (Raw8 for aligned ones).
+template <typename W>
+struct RawAny {
+  typename Vec8<W>::type v;
+  __device__ __forceinline__ void load(const W* p) {
+    v = __builtin_bit_cast(typename Vec8<W>::type, static_cast<u32x4>(*reinterpret_cast<const u32x4_any*>(p)));
+  }
+  __device__ __forceinline__ float operator[](int i) const { return to_f32(v[i]); }
+};
+template <>
+struct RawAny<float> {
+  typedef f32x4 f32x4_any __attribute__((aligned(4)));
+  f32x4 lo, hi;
+  __device__ __forceinline__ void load(const float* p) {
+    lo = *reinterpret_cast<const f32x4_any*>(p);
+    hi = *reinterpret_cast<const f32x4_any*>(p + 4);
+  }
+  __device__ __forceinline__ float operator[](int i) const { return i < 4 ? lo[i] : hi[i - 4]; }
+};
+
+template <typename T, typename W, int LPR, int VPL, int RPT, bool ADD>
+__global__ __launch_bounds__(256) void rms_rows_kernel(T* y, T* ro, const T* x, const T* r, const W* __restrict__ w,
+                                                       RowGrid grid, RowStrides lx, RowStrides lr, RowStrides ly,
+                                                       RowStrides lro, int n, uint32_t rows, float eps) {
+  typedef typename Vec8<T>::type V8;
+  constexpr int RPP = 256 / LPR;  // rows of a pass of the workgroup
+  const int l = threadIdx.x % LPR;
+  const int nv = (n + 7) / 8;
+  int k[VPL], skip[VPL];  // first element; elements the vector before it has
+  bool in[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int v = j * LPR + l;
+    in[j] = v < nv;
+    k[j] = v * 8 + 8 <= n ? v * 8 : n - 8;
+    skip[j] = v * 8 - k[j];
+  }
+  uint32_t row[RPT];
+  V8 a[RPT][VPL], b[RPT][ADD ? VPL : 1];
+#pragma unroll
+  for (int t = 0; t < RPT; ++t) {
+    row[t] = (blockIdx.x * RPT + t) * RPP + threadIdx.x / LPR;
+    const RowPos p = row_pos(grid, row[t] < rows ? row[t] : 0);
+    const T* xr = x + row_off(lx, p);
+    const T* rr = ADD ? r + row_off(lr, p) : nullptr;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      a[t][j] = load8_any<T>(xr + k[j]);
+      if constexpr (ADD) b[t][j] = load8_any<T>(rr + k[j]);
+    }
+  }
+  RawAny<W> wv[VPL];  // the lane's weights, the same for each of its rows
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) wv[j].load(w + k[j]);
+#pragma unroll
+  for (int t = 0; t < RPT; ++t) {
+    auto value = [&](int j, int i) {
+      const float f = to_f32(a[t][j][i]);
+      return ADD ? f + to_f32(b[t][ADD ? j : 0][i]) : f;
+    };
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float f = value(j, i), q = in[j] && i >= skip[j] ? f : 0.f;
+        ss += q * q;
+      }
+    if constexpr (LPR >= 64) ss = xlane_sum<32>(ss);
+    if constexpr (LPR >= 32) ss = xlane_sum<16>(ss);
+    if constexpr (LPR >= 16) ss = xlane_sum<8>(ss);
+    if constexpr (LPR >= 8) ss = xlane_sum<4>(ss);
+    if constexpr (LPR >= 4) ss = xlane_sum<2>(ss);
+    if constexpr (LPR >= 2) ss = xlane_sum<1>(ss);
+    const float inv = rsqrtf(ss / (float)n + eps);
+    const RowPos p = row_pos(grid, row[t]);
+    T* yr = y + row_off(ly, p);
+    T* ror = ADD ? ro + row_off(lro, p) : nullptr;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      V8 o, s;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float f = value(j, i);
+        o[i] = from_f32<T>(f * inv * wv[j][i]);
+        if constexpr (ADD) s[i] = from_f32<T>(f);
+      }
+      if (in[j] && row[t] < rows) {
+        if constexpr (ADD) store8_any<T>(ror + k[j], s);
+        store8_any<T>(yr + k[j], o);
+      }
+    }
+  }
+}
+
 template <typename T, bool ADD>
 __global__ __launch_bounds__(256) void rms_gen_kernel(T* y, T* ro, const T* x, const T* r,
                                                       const void* __restrict__ w, int w_dtype,
@@ -247,6 +373,42 @@ void launch_wave(void* y, void* ro, const void* x, const void* r, const void* w,
                      row_strides(ly), row_strides(lro), (int)lx.n, (uint32_t)rows, eps);
 }
 
+template <typename T, typename W, int LPR, int VPL, int RPT, bool ADD>
+void launch_rows_r(void* y, void* ro, const void* x, const void* r, const void* w, const fd_rows& lx,
+                   const fd_rows& lr, const fd_rows& ly, const fd_rows& lro, int64_t rows, float eps,
+                   hipStream_t st) {
+  constexpr int per = 256 / LPR * RPT;
+  hipLaunchKernelGGL((rms_rows_kernel<T, W, LPR, VPL, RPT, ADD>), dim3((unsigned)((rows + per - 1) / per)),
+                     dim3(256), 0, st, static_cast<T*>(y), static_cast<T*>(ro), static_cast<const T*>(x),
+                     static_cast<const T*>(r), static_cast<const W*>(w), row_grid(lx), row_strides(lx),
+                     row_strides(lr), row_strides(ly), row_strides(lro), (int)lx.n, (uint32_t)rows, eps);
+}
+
+template <typename T, typename W, bool ADD>
+void launch_rows(void* y, void* ro, const void* x, const void* r, const void* w, const fd_rows& lx,
+                 const fd_rows& lr, const fd_rows& ly, const fd_rows& lro, int64_t rows, float eps, hipStream_t st) {
+  const int64_t nv = (lx.n + 7) / 8;
+#define FD_ROWS(LPR, VPL, RPT) launch_rows_r<T, W, LPR, VPL, RPT, ADD>(y, ro, x, r, w, lx, lr, ly, lro, rows, eps, st)
+  // several rows per lane group once one each would already fill the GPU
+#define FD_ROWS_SHORT(LPR)                                            \
+  do {                                                                \
+    if (rows >= (int64_t)device_cus() * 8 * (256 / LPR)) FD_ROWS(LPR, 1, 4); else FD_ROWS(LPR, 1, 1); \
+  } while (0)
+  if (nv <= 8) FD_ROWS_SHORT(8);
+  else if (nv <= 16) FD_ROWS_SHORT(16);
+  else if (nv <= 32) FD_ROWS_SHORT(32);
+  else if (nv <= 64) FD_ROWS(64, 1, 1);
+  else if (nv <= 128) FD_ROWS(64, 2, 1);
+  else if (nv <= 192) FD_ROWS(64, 3, 1);
+  else if (nv <= 256) FD_ROWS(64, 4, 1);
+  else if (nv <= 384) FD_ROWS(64, 6, 1);
+  else if (nv <= 512) FD_ROWS(64, 8, 1);
+  else if (nv <= 768) FD_ROWS(64, 12, 1);
+  else FD_ROWS(64, 16, 1);
+#undef FD_ROWS_SHORT
+#undef FD_ROWS
+}
+
 template <typename T, typename W, bool ADD>
 void pick_vpt(void* y, void* ro, const void* x, const void* r, const void* w,
               const fd_rows& lx, const fd_rows& lr, const fd_rows& ly, const fd_rows& lro,
@@ -281,6 +443,18 @@ void pick_vpt(void* y, void* ro, const void* x, const void* r, const void* w,
 }
 
 template <typename T, bool ADD>
+void dispatch_rows_w(int w_dtype, void* y, void* ro, const void* x, const void* r, const void* w, const fd_rows& lx,
+                     const fd_rows& lr, const fd_rows& ly, const fd_rows& lro, int64_t rows, float eps,
+                     hipStream_t st) {
+  if (w_dtype == FD_F32)
+    launch_rows<T, float, ADD>(y, ro, x, r, w, lx, lr, ly, lro, rows, eps, st);
+  else if (w_dtype == FD_BF16)
+    launch_rows<T, bf16, ADD>(y, ro, x, r, w, lx, lr, ly, lro, rows, eps, st);
+  else
+    launch_rows<T, f16, ADD>(y, ro, x, r, w, lx, lr, ly, lro, rows, eps, st);
+}
+
+template <typename T, bool ADD>
 void dispatch_w(int w_dtype, void* y, void* ro, const void* x, const void* r, const void* w,
                 const fd_rows& lx, const fd_rows& lr, const fd_rows& ly, const fd_rows& lro,
                 int64_t rows, float eps, hipStream_t st) {
@@ -293,6 +467,8 @@ void dispatch_w(int w_dtype, void* y, void* ro, const void* x, const void* r, co
 }
 
 constexpr int64_t kVecMaxN = 256 * 8 * 8;
+constexpr int64_t kShortN = 256;    // rows of at most half a wave's vectors
+constexpr int64_t kRowsMaxN = 8192;  // 16 vectors of 8 per lane
 
 bool vec_ok(const void* p, const fd_rows& l, int elem) {
   return rows_vectorizable(p, l, elem) && l.n <= kVecMaxN;
@@ -316,12 +492,23 @@ int rms_common(bool add, void* y, void* ro, const void* x, const void* r, const 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const fd_rows& LR = add ? *lr : *lx;
   const fd_rows& LRO = add ? *lro : *ly;
-  const int wsz = w_dtype == FD_F32 ? 4 : 2;
   bool vec = vec_ok(x, *lx, 2) && vec_ok(y, *ly, 2) && w_stride == 1 &&
              (reinterpret_cast<uintptr_t>(w) % 16) == 0;
-  (void)wsz;
   if (add) vec = vec && vec_ok(r, *lr, 2) && vec_ok(ro, *lro, 2);
-  if (vec) {
+  // Rows of unit column stride that the wave kernels don't take, and the short
+  // rows that they take with most lanes idle.
+  const bool unit = lx->col == 1 && ly->col == 1 && (!add || (lr->col == 1 && lro->col == 1)) && w_stride == 1;
+  const bool by_rows = unit && lx->n >= 8 && lx->n <= (vec ? kShortN : kRowsMaxN);
+  if (by_rows) {
+#define FD_RMS_ROWS(T, A) \
+  dispatch_rows_w<T, A>(w_dtype, y, ro, x, r, w, *lx, LR, *ly, LRO, rows, eps, st)
+    if (act_dtype == FD_F16) {
+      if (add) FD_RMS_ROWS(f16, true); else FD_RMS_ROWS(f16, false);
+    } else {
+      if (add) FD_RMS_ROWS(bf16, true); else FD_RMS_ROWS(bf16, false);
+    }
+#undef FD_RMS_ROWS
+  } else if (vec) {
     if (act_dtype == FD_F16) {
       if (add)
         dispatch_w<f16, true>(w_dtype, y, ro, x, r, w, *lx, LR, *ly, LRO, rows, eps, st);
