@@ -81,6 +81,19 @@ __device__ __forceinline__ void store8(T* p, typename Vec8<T>::type v) {
   *reinterpret_cast<typename Vec8<T>::type*>(p) = v;
 }
 
+// The same at any element address: gfx950 moves a 2-byte aligned 16-byte word in
+// one instruction.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <typename T>
+__device__ __forceinline__ typename Vec8<T>::type load8_any(const T* p) {
+  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+  return __builtin_bit_cast(typename Vec8<T>::type, v);
+}
+template <typename T>
+__device__ __forceinline__ void store8_any(T* p, typename Vec8<T>::type v) {
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4_any*>(p));
+}
+
 // 8 consecutive values of any of the three dtypes, widened to float32.
 template <typename W>
 __device__ __forceinline__ void load8_f32(const W* p, float (&f)[8]) {
@@ -111,6 +124,24 @@ template <> struct Raw8<float> {
   __device__ __forceinline__ void load(const float* p) {
     lo = *reinterpret_cast<const f32x4*>(p);
     hi = *reinterpret_cast<const f32x4*>(p + 4);
+  }
+  __device__ __forceinline__ float operator[](int i) const { return i < 4 ? lo[i] : hi[i - 4]; }
+};
+
+// Raw8 at any element address.
+template <typename W> struct RawAny {
+  typename Vec8<W>::type v;
+  __device__ __forceinline__ void load(const W* p) {
+    v = __builtin_bit_cast(typename Vec8<W>::type, static_cast<u32x4>(*reinterpret_cast<const u32x4_any*>(p)));
+  }
+  __device__ __forceinline__ float operator[](int i) const { return to_f32(v[i]); }
+};
+template <> struct RawAny<float> {
+  typedef f32x4 f32x4_any __attribute__((aligned(4)));
+  f32x4 lo, hi;
+  __device__ __forceinline__ void load(const float* p) {
+    lo = *reinterpret_cast<const f32x4_any*>(p);
+    hi = *reinterpret_cast<const f32x4_any*>(p + 4);
   }
   __device__ __forceinline__ float operator[](int i) const { return i < 4 ? lo[i] : hi[i - 4]; }
 };

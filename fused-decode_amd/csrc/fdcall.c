@@ -88,6 +88,8 @@ static int (*p_add_rms_norm)(void*, void*, const void*, const void*, const void*
                              int, void*);
 static int (*p_swiglu)(void*, const void*, const void*, const fd_rows*, const fd_rows*,
                        const fd_rows*, int, void*);
+static int (*p_add_rows)(void*, const void*, const void*, int, const fd_rows*, const fd_rows*,
+                         const fd_rows*, int, void*);
 static int (*p_rope)(void*, const void*, const void*, const void*, int, const fd_rows*,
                      const fd_rows*, const fd_rows*, const fd_rows*, int, void*);
 static int (*p_linear_tiled)(void*, const void*, const void*, const void*, int, const void*, int,
@@ -147,6 +149,9 @@ WRAP(add_rms_norm, "pppppilrrrrfis",
 WRAP(swiglu, "ppprrris",
      p_swiglu(a[0].p, a[1].p, a[2].p, (const fd_rows*)a[3].p, (const fd_rows*)a[4].p,
               (const fd_rows*)a[5].p, a[6].i, a[7].p))
+WRAP(add_rows, "pppirrris",
+     p_add_rows(a[0].p, a[1].p, a[2].p, a[3].i, (const fd_rows*)a[4].p, (const fd_rows*)a[5].p,
+                (const fd_rows*)a[6].p, a[7].i, a[8].p))
 WRAP(rope, "ppppirrrris",
      p_rope(a[0].p, a[1].p, a[2].p, a[3].p, a[4].i, (const fd_rows*)a[5].p, (const fd_rows*)a[6].p,
             (const fd_rows*)a[7].p, (const fd_rows*)a[8].p, a[9].i, a[10].p))
@@ -227,6 +232,7 @@ static PyObject* w_bind(PyObject* self, PyObject* arg) {
   RESOLVE(p_rms_norm, "fd_rms_norm");
   RESOLVE(p_add_rms_norm, "fd_add_rms_norm");
   RESOLVE(p_swiglu, "fd_swiglu");
+  RESOLVE(p_add_rows, "fd_add_rows");
   RESOLVE(p_rope, "fd_rope");
   RESOLVE(p_linear_tiled, "fd_linear_tiled");
   RESOLVE(p_post_attn_mlp, "fd_post_attn_mlp");
@@ -253,6 +259,7 @@ static PyMethodDef methods[] = {
     FAST(rms_norm),
     FAST(add_rms_norm),
     FAST(swiglu),
+    FAST(add_rows),
     FAST(rope),
     FAST(linear_tiled),
     FAST(post_attn_mlp),

@@ -211,36 +211,6 @@ __global__ __launch_bounds__(256, !ADD && VPL <= 8 ? 8 : 1) void rms_wave_kernel
 // 15.9 -> 8.8 us, 8192 x 1025 18.5 -> 9.7, 4096 x 8191 68.8 -> 27.0, 65536 x 100 42.0
 // -> 6.9, one row of 4097 6.1 -> 4.3. Aligned rows past 256 stay with the wave kernel,
 // whose weights sit in LDS (4096 x 8192 23.0 us).
-typedef u32x4 u32x4_any __attribute__((aligned(2)));
-template <typename T>
-__device__ __forceinline__ typename Vec8<T>::type load8_any(const T* p) {
-  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
-  return __builtin_bit_cast(typename Vec8<T>::type, v);
-}
-template <typename T>
-__device__ __forceinline__ void store8_any(T* p, typename Vec8<T>::type v) {
-  __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4_any*>(p));
-}
-// 8 norm weights at any address, in their storage form (Raw8 for aligned ones).
-template <typename W>
-struct RawAny {
-  typename Vec8<W>::type v;
-  __device__ __forceinline__ void load(const W* p) {
-    v = __builtin_bit_cast(typename Vec8<W>::type, static_cast<u32x4>(*reinterpret_cast<const u32x4_any*>(p)));
-  }
-  __device__ __forceinline__ float operator[](int i) const { return to_f32(v[i]); }
-};
-template <>
-struct RawAny<float> {
-  typedef f32x4 f32x4_any __attribute__((aligned(4)));
-  f32x4 lo, hi;
-  __device__ __forceinline__ void load(const float* p) {
-    lo = *reinterpret_cast<const f32x4_any*>(p);
-    hi = *reinterpret_cast<const f32x4_any*>(p + 4);
-  }
-  __device__ __forceinline__ float operator[](int i) const { return i < 4 ? lo[i] : hi[i - 4]; }
-};
-
 template <typename T, typename W, int LPR, int VPL, int RPT, bool ADD>
 __global__ __launch_bounds__(256) void rms_rows_kernel(T* y, T* ro, const T* x, const T* r, const W* __restrict__ w,
                                                        RowGrid grid, RowStrides lx, RowStrides lr, RowStrides ly,

@@ -65,6 +65,7 @@ SIGNATURES: dict[str, list] = {
     "fd_rms_norm": [_p, _p, _p, _i, _l, _rows, _rows, _f, _i, _p],
     "fd_add_rms_norm": [_p, _p, _p, _p, _p, _i, _l, _rows, _rows, _rows, _rows, _f, _i, _p],
     "fd_swiglu": [_p, _p, _p, _rows, _rows, _rows, _i, _p],
+    "fd_add_rows": [_p, _p, _p, _i, _rows, _rows, _rows, _i, _p],
     "fd_rope": [_p, _p, _p, _p, _i, _rows, _rows, _rows, _rows, _i, _p],
     "fd_linear": [_p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _i, _i, _p],
     "fd_linear_fp8": [_p, _p, _p, _p, _p, _i, _p, _i, _l, _l, _l, _l, _l, _l, _l, _l, _l, _l, _i, _p],

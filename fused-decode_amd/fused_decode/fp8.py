@@ -23,12 +23,11 @@ import math
 import warnings
 
 import torch
-from torch.autograd import forward_ad
 
 from . import _lib
 from ._checks import check
 from ._lib import DTYPE_CODE, fail, native
-from .ops import (_FP8_ROWS, _PLANS, _check_out, _dense, _empty, _plan_qkv, _raw_stream, _remember, _row_add_rows,
+from .ops import (_FP8_ROWS, _PLANS, _check_out, _dense, _empty, _only_values, _plan_qkv, _raw_stream, _remember, _row_add_rows,
                   _sig, rms_norm, swiglu)
 
 FP8_MAX = 448.0
@@ -45,20 +44,6 @@ def _slow_path(why: str) -> None:
         warnings.warn(f"linear_decode_fp8: {why}; computing a float32 product of the decoded weights "
                       "(same values, about 4x the weight traffic of the fp8 kernels)", RuntimeWarning,
                       stacklevel=5)  # _slow_path, the plan's helper, the plan, linear_decode_fp8, its caller
-
-
-def _only_values(*tensors) -> bool:
-    """Whether these are plain tensors that nothing records or transforms, so that a
-    launch on their pointers says all that the torch formula would: no gradient
-    wanted, no forward-mode level, no vmap or tracing."""
-    if forward_ad._current_level >= 0 or torch.compiler.is_compiling():
-        return False
-    grad = torch.is_grad_enabled()
-    for t in tensors:
-        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)
-                              or torch._C._functorch.is_functorch_wrapped_tensor(t)):
-            return False
-    return True
 
 
 def quantize_fp8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:

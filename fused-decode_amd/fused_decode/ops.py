@@ -33,11 +33,12 @@ from typing import Callable, NamedTuple
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._checks import check
 from ._layout import contiguous_strides, plan_rows
-from ._lib import DTYPE_CODE, FD_EUNSUPPORTED, KIND_CODE, FdTile, fail, native
+from ._lib import DTYPE_CODE, FD_EUNSUPPORTED, KIND_CODE, FdRows, FdTile, fail, native
 from .kernels import (
     _rms_env,
     linear_config,
@@ -134,6 +135,20 @@ def _empty(shape, like: torch.Tensor) -> Callable[[torch.Tensor], torch.Tensor]:
         return torch.empty_like
     dtype, device = like.dtype, like.device
     return lambda _ref: torch.empty(shape, dtype=dtype, device=device)
+
+
+def _only_values(*tensors) -> bool:
+    """Whether these are plain tensors that nothing records or transforms, so that a
+    launch on their pointers says all that the torch formula would: no gradient
+    wanted, no forward-mode level, no vmap or tracing."""
+    if forward_ad._current_level >= 0 or torch.compiler.is_compiling():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)
+                              or torch._C._functorch.is_functorch_wrapped_tensor(t)):
+            return False
+    return True
 
 
 # ------------------------------------------------------------------ norms
@@ -462,10 +477,29 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
         return x2, r.expand(expected).reshape(m, n)
 
     if m > limit:  # hipBLASLt, bit-identical to F.linear; row_add in float32, one rounding
+        dense = bytes(FdRows(1, 1, m, 0, 0, n, 1, n))
+        if ra is not None:
+            add_rows, act, dev = native().add_rows, DTYPE_CODE[x.dtype], x.device.index
+            r_rows, rcode = bytes(FdRows(1, 1, m, 0, 0, ra[0], ra[1], n)), DTYPE_CODE[row_add.dtype]
+
         def fallback(x, w, b, r, out):
             x2, r2 = operands(x, r)
             y = F.linear(x2, w, b)
-            if r2 is not None:
+            if r2 is not None and y.dtype == x.dtype and y.is_contiguous() and _only_values(x, w, b, r):
+                if ra[2]:
+                    r = r.expand(expected).reshape(m, n)
+                # straight into `out`, unless r might be part of it
+                direct = out is not None and out.untyped_storage().data_ptr() != r.untyped_storage().data_ptr()
+                status = add_rows((out if direct else y).data_ptr(), y.data_ptr(), r.data_ptr(), rcode, dense, r_rows,
+                                  dense, act, _raw_stream(dev))
+                if status == 0:
+                    if direct:
+                        return out
+                elif status == FD_EUNSUPPORTED:
+                    y = (y.float() + r2.float()).to(x.dtype)
+                else:
+                    fail("fd_add_rows", status)
+            elif r2 is not None:
                 y = (y.float() + r2.float()).to(x.dtype)
             if out is None:
                 return y.view(expected)

@@ -103,6 +103,16 @@ int fd_swiglu(void* y, const void* gate, const void* up, const fd_rows* lg,
               const fd_rows* lu, const fd_rows* ly, int act_dtype, void* stream);
 
 /*
+ * y = round(a + r) in float32: the row_add of a product that is already in
+ * memory (linear_decode above the GEMV's rows, kernels.py:657-672). a and y are
+ * rows of unit column stride; r has any strides (0 = broadcast) and any of the
+ * three dtypes. y may be a. Replaces no reference launcher (it adds in PyTorch,
+ * ops.py:273-278).
+ */
+int fd_add_rows(void* y, const void* a, const void* r, int r_dtype, const fd_rows* la,
+                const fd_rows* lr, const fd_rows* ly, int act_dtype, void* stream);
+
+/*
  * Rotate-half RoPE over rows of even length n, h = n/2:
  *   y[:h] = x1*c1 - x2*s1,  y[h:] = x2*c2 + x1*s2   (float32, one rounding).
  * cos/sin rows (dtype cs_dtype: FD_F16, FD_BF16 or FD_F32) use their own layouts,
