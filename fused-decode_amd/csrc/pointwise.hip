@@ -6,6 +6,7 @@
 // the activations (each byte is touched once); the generic kernels take any
 // column stride and any row length.
 #include "fd_device.h"
+#include "fd_gemv.h"
 #include "fd_host.h"
 
 namespace fd {
@@ -28,23 +29,40 @@ __device__ __forceinline__ void store8_from(T* p, const typename Vec8<T>::type& 
 // SwiGLU: y = round(silu(g) * u), float32 math (reference.py:33-35, stable sigmoid
 // as kernels.py:448-451).
 
-template <typename T>
+//
+// Rows of unit column stride at any element address (one 16-byte word per operand
+// and thread, aligned or not). Where n % 8 != 0 a row's last thread loads the 8
+// elements up to its end and stores only those past the thread before it, so that
+// no element one thread writes matters to another (the operation may be in place).
+// Rows of 14335 by this kernel and element by element: 2048 of them 35.9 and 79.3
+// us (14336: 29.6), 64 3.4 and 3.8, one 2.2 and 1.9; 2048 x 1025 4.6 and 7.0.
+// ALIGNED (rows of whole, 16-byte aligned vectors) leaves the last thread's case
+// out, which costs 1.2% at 2048 x 14336.
+template <typename T, bool ALIGNED>
 __global__ __launch_bounds__(kPwThreads) void swiglu_vec_kernel(T* y, const T* g, const T* u,
                                                                 RowGrid grid, FastDiv vpr,
                                                                 RowStrides sg, RowStrides su,
-                                                                RowStrides sy, uint32_t total) {
+                                                                RowStrides sy, uint32_t total, uint32_t n) {
   const uint32_t v = blockIdx.x * kPwThreads + threadIdx.x;
   if (v >= total) return;
   uint32_t cv;
   const uint32_t row = vpr.divmod(v, cv);
-  const uint32_t k = cv * 8;
+  const uint32_t k = ALIGNED || cv * 8 + 8 <= n ? cv * 8 : n - 8;
   const RowPos p = row_pos(grid, row);
-  typename Vec8<T>::type a = load8_nt<T>(g + row_off(sg, p) + k);
-  typename Vec8<T>::type b = load8_nt<T>(u + row_off(su, p) + k);
-  typename Vec8<T>::type o;
+  typename Vec8<T>::type a, b, o;
+  if constexpr (ALIGNED) {
+    a = load8_nt<T>(g + row_off(sg, p) + k);
+    b = load8_nt<T>(u + row_off(su, p) + k);
+  } else {
+    a = load8_any<T>(g + row_off(sg, p) + k);
+    b = load8_any<T>(u + row_off(su, p) + k);
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[i] = from_f32<T>(silu_stable(to_f32(a[i])) * to_f32(b[i]));
-  store8_nt<T>(y + row_off(sy, p) + k, o);
+  if constexpr (ALIGNED)
+    store8_nt<T>(y + row_off(sy, p) + k, o);
+  else
+    store8_from<T>(y + row_off(sy, p) + k, o, cv * 8 - k);
 }
 
 template <typename T>
@@ -66,10 +84,8 @@ __global__ __launch_bounds__(kPwThreads) void swiglu_gen_kernel(T* y, const T* g
 // y = round(a + r) in float32: the residual of a product that another library
 // wrote (row_add above the GEMV's rows, kernels.py:657-672 order), in one pass
 // where float32 copies of both operands, their sum and its rounding take four
-// (777 x 4096 float16: 27 -> 5.7 us). a and y are rows of unit column stride at
-// any element address, r may have any strides (0 = broadcast) and dtype. Where n % 8
-// != 0 a row's last thread loads the 8 elements up to its end and stores only those
-// past the thread before it (y may be a).
+// (777 x 4096 float16: 27 -> 5.7 us). Rows as swiglu_vec_kernel's; r may
+// have any strides (0 = broadcast) and dtype.
 template <typename T, typename R>
 __global__ __launch_bounds__(kPwThreads) void add_rows_kernel(T* y, const T* a, const R* r, RowGrid grid,
                                                               FastDiv vpr, RowStrides sa, RowStrides sr,
@@ -209,16 +225,24 @@ extern "C" int fd_swiglu(void* y, const void* gate, const void* up, const fd_row
   if (total > kMaxPwWork) return set_error(FD_EUNSUPPORTED, "swiglu tensor too large (>= 2^32 elements)");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const RowGrid grid = row_grid(*lg);
-  const bool vec = rows_vectorizable(gate, *lg, 2) && rows_vectorizable(up, *lu, 2) &&
-                   rows_vectorizable(y, *ly, 2);
+  const bool aligned = rows_vectorizable(gate, *lg, 2) && rows_vectorizable(up, *lu, 2) &&
+                       rows_vectorizable(y, *ly, 2);
+  // other rows in vectors too once these make a workgroup for every CU; below,
+  // the per-element kernel's eight times as many threads finish sooner
+  const bool vec = aligned || (lg->col == 1 && lu->col == 1 && ly->col == 1 && lg->n >= 8 &&
+                               total >= (int64_t)8 * kPwThreads * device_cus());
   if (vec) {
-    const uint32_t tv = (uint32_t)(total / 8);
-    const FastDiv vpr((uint32_t)(lg->n / 8));
-#define FD_SWIGLU_VEC(T)                                                                       \
-  hipLaunchKernelGGL(swiglu_vec_kernel<T>, dim3(blocks_for(tv)), dim3(kPwThreads), 0, st,      \
+    const uint32_t vectors = (uint32_t)((lg->n + 7) / 8), tv = (uint32_t)rows * vectors;
+    const FastDiv vpr(vectors);
+#define FD_SWIGLU_VEC(T, A)                                                                    \
+  hipLaunchKernelGGL((swiglu_vec_kernel<T, A>), dim3(blocks_for(tv)), dim3(kPwThreads), 0, st, \
                      (T*)y, (const T*)gate, (const T*)up, grid, vpr, row_strides(*lg),         \
-                     row_strides(*lu), row_strides(*ly), tv)
-    if (act_dtype == FD_F16) FD_SWIGLU_VEC(f16); else FD_SWIGLU_VEC(bf16);
+                     row_strides(*lu), row_strides(*ly), tv, (uint32_t)lg->n)
+    if (act_dtype == FD_F16) {
+      if (aligned) FD_SWIGLU_VEC(f16, true); else FD_SWIGLU_VEC(f16, false);
+    } else {
+      if (aligned) FD_SWIGLU_VEC(bf16, true); else FD_SWIGLU_VEC(bf16, false);
+    }
 #undef FD_SWIGLU_VEC
   } else {
     const FastDiv nd((uint32_t)lg->n);
