@@ -479,4 +479,13 @@ int launch_dma_default(unsigned blocks, void* y, const void* x, const void* w, c
   return launch_dma_rows<T, W, 2, 2, EPI, NORM>(blocks, y, x, w, ws, M, N, K, sxm, swn, sym, syn, e, r, fn, st);
 }
 
+// GEMV in workgroups of 8, 24 or 32 weight rows in place of the 16 of the kernel
+// above (gemv_oct.hip). oct_rows: the rows that a launch of M by N x K with weights
+// of `wbytes` bytes takes there, or 0 where 16 are better; `sums`: with row sums
+// (Epi::ss). launch_oct is instantiated for T = fp16 and bf16 with W = T and E4M3 codes.
+int oct_rows(int M, int N, int K, int wbytes, bool sums);
+template <typename T, typename W>
+int launch_oct(int rows, int M, void* y, const void* x, const void* w, const float* ws, int N, int K, int64_t sxm,
+               int64_t swn, int64_t sym, int64_t syn, const Epi& e, hipStream_t st);
+
 }  // namespace fd

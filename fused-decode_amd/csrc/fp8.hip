@@ -959,6 +959,8 @@ int launch_gemv_fp8_mfma(int M, void* y, const void* x, const uint8_t* w, const 
   if (rp)
     return launch_dma_default<T, uint8_t, EPI_ROPE, false>(blocks, y, x, w, s, M, N, K, sxm, swn, sym, syn, e,
                                                            *rp, nofold, st);
+  if (const int rows = oct_rows(M, N, K, 1, e.ss != nullptr))
+    return launch_oct<T, uint8_t>(rows, M, y, x, w, s, N, K, sxm, swn, sym, syn, e, st);
   if ((K + kUnit - 1) / kUnit < 4)
     return launch_dma_rows<T, uint8_t, 2, 2, EPI_PLAIN, false>(blocks, y, x, w, s, M, N, K, sxm, swn, sym, syn,
                                                                e, none, nofold, st);
