@@ -372,20 +372,34 @@ int wide_launch(const WideArgs& a, int splits) {
   return FD_OK;
 }
 
-// Tiles of 128 weight rows by the rows rounded up to 32, 64 or 128, with as many
-// stages as the LDS holds. Gate/up at those widths: 32 rows 25.0 us (31.1 in the
-// tile of 64, 40.6 in that of 128), 64 rows 28.0 (39.6, 38.6), 120 rows 39.2
-// (73.5 in four tiles of 32, 48.1 in two of 64); tiles of 64 weight rows read the
-// activations twice as often (26.4, 33.6, 50.5) and two waves a SIMD beat one
-// with twice the tile (120 rows: 39.2 against 41.4 and 47.4).
-template <typename T, int EPI>
-int wide_rows(const WideArgs& a, int splits) {
-  if (a.M <= 32) return wide_launch<T, 4, 1, 2, 2, 6, EPI>(a, splits);
-  if (a.M <= 64) return wide_launch<T, 2, 2, 4, 2, 4, EPI>(a, splits);
-  return wide_launch<T, 2, 2, 4, 4, 3, EPI>(a, splits);
+// Activation rows of a tile: 32, 64, 96 or 128, whichever takes the least time for
+// all M rows. A tile's time is about that of its rows and 74 more (gate/up at the
+// widths of Llama-3-8B: 25.0, 28.0, 33.4 and 39.2 us with one tile of 32, 64, 96 and 128
+// a weight tile). Gate/up of 32 rows 25.0 us (31.1 in the tile of 64, 40.6 in that of
+// 128), 64 rows 28.0 (39.6, 38.6), 96 rows 33.4 (40.9 in that of 128), 120 rows 39.2
+// (73.5 in four tiles of 32, 48.1 in two of 64), 192 rows 60.8 in two of 96 (71.7 in
+// two of 128), 288 rows 90.5 in three (105.8).
+inline int wide_bm(int64_t M) {
+  auto cost = [&](int64_t bm) { return (M + bm - 1) / bm * (bm + 74); };
+  int best = 32;
+  for (int bm : {64, 96, 128})
+    if (cost(bm) < cost(best)) best = bm;
+  return best;
 }
 
-inline int wide_bm(int64_t M) { return M <= 32 ? 32 : M <= 64 ? 64 : 128; }
+// Tiles of 128 weight rows, with as many stages as the LDS holds. Tiles of 64
+// weight rows read the activations twice as often (gate/up of 32, 64 and 120 rows
+// 26.4, 33.6, 50.5 us) and two waves a SIMD beat one with twice the tile (120 rows:
+// 39.2 against 41.4 and 47.4).
+template <typename T, int EPI>
+int wide_rows(const WideArgs& a, int splits) {
+  switch (wide_bm(a.M)) {
+    case 32: return wide_launch<T, 4, 1, 2, 2, 6, EPI>(a, splits);
+    case 64: return wide_launch<T, 2, 2, 4, 2, 4, EPI>(a, splits);
+    case 96: return wide_launch<T, 2, 2, 4, 3, 4, EPI>(a, splits);
+    default: return wide_launch<T, 2, 2, 4, 4, 3, EPI>(a, splits);
+  }
+}
 
 // K splits of a product: enough for one workgroup on every CU, each with at
 // least four stages, which is where the next split's sums cost what its share

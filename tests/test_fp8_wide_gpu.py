@@ -53,6 +53,15 @@ def test_linear_fp8_wide(dtype, m, n, k):
     check_product(out, wide, q, s, None, row[:1])
 
 
+@pytest.mark.parametrize("m", [66, 96, 97, 192, 193, 288])
+def test_rows_around_tiles_of_96(m):
+    import fused_decode as fd
+
+    x, (q, s) = rnd(m, 1040, seed=m, dtype=torch.bfloat16), fd.quantize_fp8(rnd(130, 1040, seed=15, scale=0.03))
+    row = rnd(m, 130, seed=16, dtype=torch.bfloat16)
+    check_product(fd.linear_decode_fp8(x, q, s, row_add=row), x, q, s, None, row)
+
+
 def test_scratch_lowers_the_split():
     """The library's preferred split, less scratch, and none: the same product."""
     import fused_decode as fd
