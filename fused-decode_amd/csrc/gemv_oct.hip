@@ -207,7 +207,7 @@ int launch_oct(int rows, int M, void* y, const void* x, const void* w, const flo
   }
   if (rows == 24) {
     if constexpr (sizeof(W) == 1)
-      if (few && (N + 23) / 24 <= device_cus()) FD_RUN(3, 8, 8);
+      if (few && ((int64_t)N + 23) / 24 <= device_cus()) FD_RUN(3, 8, 8);
     if (few) FD_RUN(3, 4, 8); else FD_RUN(3, 4, 16);
   }
   if constexpr (sizeof(W) == 1)
