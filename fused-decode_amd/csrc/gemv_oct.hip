@@ -141,7 +141,9 @@ __global__ __launch_bounds__(NW * kWave) void gemv_mfma_oct_kernel(T* y, const T
 #pragma unroll
   for (int n = 0; n < TILES; ++n) part[n][wave * kWave + lane] = acc[n];
   __syncthreads();
-  if (wave >= TILES) return;
+  // the last workgroup's second tile may start past N: it has no output rows, and no
+  // row of sums either (Epi::ss holds ceil(N / 16) of them)
+  if (wave >= TILES || nt0 >= N) return;
   f32x4 s = part[tile][lane];
   for (int i = 1; i < NW; ++i) s += part[tile][i * kWave + lane];
   mfma_tile_out_plain<T, F8>(y, s, lane, nt0, e, tep, M, (int)nend, sym, syn);

@@ -64,3 +64,22 @@ def test_row_sums(m, n):
     want = torch.zeros_like(ss)
     want[:, :m] = y.float().square().view(m, -1, 16).sum(-1).t()
     torch.testing.assert_close(ss, want, rtol=1e-5, atol=0)  # sixteen positive float32 terms
+
+
+@pytest.mark.parametrize("m", [5, 16])
+@pytest.mark.parametrize("n", [5616, 5610, 5600, 5593])  # 351 tiles of 16 (a last workgroup of one), 350; whole, ragged
+def test_row_sums_end_at_the_last_tile(m, n):
+    """The sums are the front of a longer buffer, whose rest keeps its values."""
+    from fused_decode.rowsq import linear_fp8_sumsq
+
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    x, tiles = rnd(g, m, 1024, dtype=torch.bfloat16), -(-n // 16)
+    w8, scale = codes(rnd(g, n, 1024, dtype=torch.bfloat16, scale=1024 ** -0.5))
+    y, buf = torch.empty(m, n, device="cuda", dtype=torch.bfloat16), torch.full((tiles + 4, 16), -1.0, device="cuda")
+    linear_fp8_sumsq(x, w8, scale, out=y, ss_out=buf[:tiles])
+    check(y, x.double() @ w8.double().t() * scale.double(), torch.bfloat16)
+    want = torch.full_like(buf, -1.0)
+    want[:tiles] = 0
+    sq = torch.nn.functional.pad(y.float().square(), (0, tiles * 16 - n))
+    want[:tiles, :m] = sq.view(m, tiles, 16).sum(-1).t()
+    torch.testing.assert_close(buf, want, rtol=1e-5, atol=0)  # sixteen positive float32 terms
