@@ -416,7 +416,9 @@ int wide_splits(int64_t M, int64_t N, int64_t K) {
 int wide_check(const void* x, const void* w8, int64_t M, int64_t N, int64_t K, int64_t sxm, int64_t swn) {
   if (K % 16 != 0 || !aligned16(x) || !aligned16(w8) || (M > 1 && sxm % 8 != 0) || (N > 1 && swn % 16 != 0))
     return set_error(FD_EUNSUPPORTED, "the fp8 kernels need K %% 16 == 0 and 16-byte aligned rows");
-  if (M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffff00LL) return set_error(FD_EUNSUPPORTED, "too large");
+  // the kernel's int indexes run to the end of the last tile of 128 rows and stage of 128 k
+  if (M > 0x7fffffffLL - 128 || N > 0x7fffffffLL - 128 || K > 0x7fffff00LL)
+    return set_error(FD_EUNSUPPORTED, "too large");
   return FD_OK;
 }
 

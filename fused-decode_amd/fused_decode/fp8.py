@@ -26,7 +26,7 @@ import torch
 
 from . import _lib
 from ._checks import check
-from ._lib import DTYPE_CODE, fail, native
+from ._lib import DTYPE_CODE, FD_EUNSUPPORTED, fail, native
 from .ops import (_FP8_ROWS, _PLANS, _check_out, _dense, _empty, _only_values, _plan_qkv, _raw_stream, _remember, _row_add_rows,
                   _sig, rms_norm, swiglu)
 
@@ -167,6 +167,8 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
                                bcode, None if r is None else r.data_ptr(), rcode, m, n, k, sxm, int(w.stride(0)), sb,
                                srm, srn, n, 1, None if part is None else part.data_ptr(), scratch_bytes, act,
                                _raw_stream(dev))
+            if status == FD_EUNSUPPORTED:
+                return slow(x2, w, sc, b, r, y, "the kernels' index range ends below these sizes")
             if status:
                 fail("fd_linear_fp8_wide", status)
             return y
@@ -213,10 +215,12 @@ def _plan_mlp_fp8(hidden, norm_weight, w_gate_up, gate_up_scale, w_down, down_sc
     h, i = int(w_gate_up.shape[1]), int(w_down.shape[1])
     m = hidden.numel() // h if h else 0
 
-    def composed(x, nw, wgu, sgu, wd, sd):
-        normed = rms_norm(x, nw, eps=eps)
+    def products(x, normed, wgu, sgu, wd, sd):
         gate, up = linear_decode_fp8(normed, wgu, sgu).split(i, dim=-1)
         return linear_decode_fp8(swiglu(gate, up), wd, sd, row_add=x)
+
+    def composed(x, nw, wgu, sgu, wd, sd):
+        return products(x, rms_norm(x, nw, eps=eps), wgu, sgu, wd, sd)
 
     if not (m > 0 and w_gate_up.is_contiguous() and w_down.is_contiguous() and h % 16 == 0
             and i % 16 == 0) or (m > _HAND_LIMIT and i == 0):
@@ -230,11 +234,12 @@ def _plan_mlp_fp8(hidden, norm_weight, w_gate_up, gate_up_scale, w_down, down_sc
         def wide(x, nw, wgu, sgu, wd, sd):
             normed = rms_norm(x, nw, eps=eps)
             if wgu.data_ptr() % 16 or not _only_values(normed, sgu):
-                gate, up = linear_decode_fp8(normed, wgu, sgu).split(i, dim=-1)
-                return linear_decode_fp8(swiglu(gate, up), wd, sd, row_add=x)
+                return products(x, normed, wgu, sgu, wd, sd)
             mid = normed.new_empty(mid_shape)
             status = gate_up(mid.data_ptr(), normed.data_ptr(), wgu.data_ptr(),
                              (sgu if dense_s else sgu.contiguous()).data_ptr(), m, h, i, h, act_w, _raw_stream(dev_w))
+            if status == FD_EUNSUPPORTED:  # sizes past the kernel's index range
+                return products(x, normed, wgu, sgu, wd, sd)
             if status:
                 fail("fd_gate_up_fp8_wide", status)
             return linear_decode_fp8(mid, wd, sd, row_add=x)
@@ -251,7 +256,7 @@ def _plan_mlp_fp8(hidden, norm_weight, w_gate_up, gate_up_scale, w_down, down_sc
         mid = x2.new_empty((m, i))
         status = call(y.data_ptr(), mid.data_ptr(), x2.data_ptr(), nw2.data_ptr(), nwc, wgu.data_ptr(),
                       sgu.data_ptr(), wd.data_ptr(), sd.data_ptr(), m, h, i, eps, act, _raw_stream(dev))
-        if status == _lib.FD_EUNSUPPORTED:  # e.g. an unaligned operand or a hidden width beyond the LDS
+        if status == FD_EUNSUPPORTED:  # e.g. an unaligned operand or a hidden width beyond the LDS
             return composed(x, nw, wgu, sgu, wd, sd)
         if status:
             fail("fd_post_attn_mlp_fp8", status)

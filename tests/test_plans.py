@@ -1,0 +1,72 @@
+"""Which path a launch plan takes, on CPU tensors: the library's calls are replaced by ones that only note their
+name and return a status, and the argument contract's device rule is left out."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fused_decode import fp8, ops
+from fused_decode._lib import FD_EUNSUPPORTED, FD_OK
+
+
+class Calls(list):
+    """Stands in for the native binding: notes each call and returns `status[name]` (FD_OK)."""
+
+    def __init__(self):
+        super().__init__()
+        self.status = {}
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.append(name)
+            return self.status.get(name, FD_OK)
+        return call
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    stand_in = Calls()
+    for mod in (ops, fp8):
+        monkeypatch.setattr(mod, "native", lambda: stand_in)
+        monkeypatch.setattr(mod, "check", lambda op, **a: a)
+        monkeypatch.setattr(mod, "_raw_stream", lambda dev: 0)
+    monkeypatch.setattr(fp8, "_warned", set())
+    ops.clear_plans()
+    yield stand_in
+    ops.clear_plans()
+
+
+def rnd(*shape, seed, dtype=torch.float32):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def fp8_case(m=20, n=32, k=64):
+    x, (q, s) = rnd(m, k, seed=1, dtype=torch.bfloat16), fp8.quantize_fp8(rnd(n, k, seed=2))
+    return x, q, s
+
+
+def product(x, q, s, row=0.0):
+    return ((x.float() @ q.float().t()) * s + row).to(x.dtype)
+
+
+def test_sizes_that_the_wide_kernels_refuse_are_still_computed(calls):
+    x, q, s = fp8_case()
+    fp8.linear_decode_fp8(x, q, s)
+    assert calls == ["linear_fp8_wide"]
+    calls.status["linear_fp8_wide"] = FD_EUNSUPPORTED
+    with pytest.warns(RuntimeWarning, match="index range"):
+        y = fp8.linear_decode_fp8(x, q, s)
+    assert torch.equal(y, product(x, q, s))
+
+
+def test_an_mlp_whose_gate_up_is_refused_is_composed(calls):
+    x, (gu, gs), (d, ds) = rnd(20, 64, seed=1, dtype=torch.bfloat16), *(fp8.quantize_fp8(rnd(*s, seed=i))
+                                                                      for i, s in enumerate(((64, 64), (64, 32))))
+    run = lambda: fp8.post_attn_mlp_fp8(x, torch.ones(64), gu, gs, d, ds)
+    run()
+    assert calls == ["rms_norm", "gate_up_fp8_wide", "linear_fp8_wide"]
+    calls.clear()
+    calls.status["gate_up_fp8_wide"] = FD_EUNSUPPORTED
+    run()
+    assert calls == ["rms_norm", "gate_up_fp8_wide", "linear_fp8_wide", "swiglu", "linear_fp8_wide"]

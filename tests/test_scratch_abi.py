@@ -26,6 +26,24 @@ def test_wide_entry_points_reject():
     assert gate(x=None) == L.FD_EINVAL and gate(h=120) == L.FD_EUNSUPPORTED and gate(m=0) == L.FD_OK
 
 
+def test_wide_sizes_end_below_the_index_range():
+    """The kernel's 32-bit indexes reach the end of the last tile, up to 127 rows past M and N."""
+    from fused_decode import _lib as L
+
+    lib, top = L.lib(), 2**31 - 1
+    refused = lambda status: status == L.FD_EUNSUPPORTED and b"too large" in lib.fd_last_error()
+
+    def lin(m, n):
+        return lib.fd_linear_fp8_wide(FAKE, FAKE, FAKE, FAKE, None, 0, None, 0, m, n, 128, 128, 128, 0, 0, 0, n, 1, None,
+                                      0, 0, None)
+
+    for past in (top - 127, top - 15, top, top + 1):
+        assert refused(lin(32, past)) and refused(lin(past, 64))
+    half = (top + 1) // 2  # gate/up: 2 I weight rows
+    for i in (half - 63, half):
+        assert refused(lib.fd_gate_up_fp8_wide(FAKE, FAKE, FAKE, FAKE, 32, 128, i, 128, 0, None))
+
+
 def test_wide_scratch_follows_the_tiles():
     """No split, so no scratch, once the output tiles cover the GPU; else float32 sums for each split."""
     from fused_decode import _lib as L
