@@ -64,6 +64,26 @@ inline bool overlaps(const void* a, int64_t na, const void* b, int64_t nb) {
   return na > 0 && nb > 0 && pa < pb + (uintptr_t)nb && pb < pa + (uintptr_t)na;
 }
 
+// Bytes from the first to past the last of rows x cols elements at r * sr + c * sc
+// (strides >= 0).
+inline int64_t span_bytes(int64_t rows, int64_t cols, int64_t sr, int64_t sc, int64_t elem_bytes) {
+  return rows > 0 && cols > 0 ? ((rows - 1) * sr + (cols - 1) * sc + 1) * elem_bytes : 0;
+}
+
+inline int dtype_bytes(int dt) { return dt == FD_F32 ? 4 : 2; }
+
+// True when an epilogue that reads row_add at other elements than the one it then
+// writes could meet the output: row_add [M,N] and y share memory, and row_add is not
+// y's own elements in y's order.
+inline bool row_add_meets(const void* row_add, int row_dtype, int64_t srm, int64_t srn, const void* y, int act_dtype,
+                          int64_t sym, int64_t syn, int64_t M, int64_t N) {
+  if (!row_add || !overlaps(row_add, span_bytes(M, N, srm, srn, dtype_bytes(row_dtype)), y,
+                            span_bytes(M, N, sym, syn, dtype_bytes(act_dtype))))
+    return false;
+  const bool same = row_add == y && row_dtype == act_dtype && (M == 1 || srm == sym) && (N == 1 || srn == syn);
+  return !same;
+}
+
 // The MLP entry points write y and mid while hidden is still to be read (the
 // down projection adds hidden as its residual, and from M = 5 y first holds the
 // normalised rows): none of the three may share memory.

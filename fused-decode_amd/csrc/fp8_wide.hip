@@ -453,6 +453,13 @@ extern "C" int fd_linear_fp8_wide(void* y, const void* x, const void* w8, const 
   if (!y || !x || !w8 || !w_scale) return set_error(FD_EINVAL, "null pointer argument");
   int rc = wide_check(x, w8, M, N, K, sxm, swn);
   if (rc != FD_OK) return rc;
+  // tiles are stored while other workgroups still read their operands
+  const int64_t ny = span_bytes(M, N, sym, syn, 2);
+  if (overlaps(y, ny, x, span_bytes(M, K, sxm, 1, 2)) || overlaps(y, ny, w8, span_bytes(N, K, swn, 1, 1)) ||
+      overlaps(y, ny, w_scale, N * 4) ||
+      (bias && overlaps(y, ny, bias, span_bytes(1, N, 0, sb, dtype_bytes(bias_dtype)))) ||
+      row_add_meets(row_add, row_dtype, srm, srn, y, act_dtype, sym, syn, M, N))
+    return set_error(FD_EUNSUPPORTED, "y must not overlap an operand, other than as row_add itself");
   const int64_t quads = (N + 3) / 4;
   int splits = wide_splits(M, N, K);
   if (!scratch) scratch_bytes = 0;
@@ -495,6 +502,10 @@ extern "C" int fd_gate_up_fp8_wide(void* mid, const void* x, const void* w_gate_
   if (!mid || !x || !w_gate_up8 || !gate_up_scale) return set_error(FD_EINVAL, "null pointer argument");
   int rc = wide_check(x, w_gate_up8, M, 2 * I, H, sxm, H);
   if (rc != FD_OK) return rc;
+  const int64_t nm = M * I * 2;  // stored while other workgroups still read
+  if (overlaps(mid, nm, x, span_bytes(M, H, sxm, 1, 2)) || overlaps(mid, nm, w_gate_up8, 2 * I * H) ||
+      overlaps(mid, nm, gate_up_scale, 2 * I * 4))
+    return set_error(FD_EINVAL, "mid must not overlap x or the weights");
   WideArgs a{mid, nullptr, x,     static_cast<const uint8_t*>(w_gate_up8), gate_up_scale, (int)M, (int)(2 * I), (int)H, sxm,
              H,   I,       1,     Epi{}, static_cast<hipStream_t>(stream)};
   rc = act_dtype == FD_F16 ? wide_rows<f16, WIDE_SWIGLU>(a, 1) : wide_rows<bf16, WIDE_SWIGLU>(a, 1);

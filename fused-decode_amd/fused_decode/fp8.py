@@ -162,11 +162,20 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
             r = r.expand(expected).reshape(m, n)
         if wide:
             part = x2.new_empty(scratch_bytes // 4, dtype=torch.float32) if scratch_bytes else None
-            status = call_wide(y.data_ptr(), x2.data_ptr(), w.data_ptr(),
-                               (sc if dense_sc else sc.contiguous()).data_ptr(), None if b is None else b.data_ptr(),
-                               bcode, None if r is None else r.data_ptr(), rcode, m, n, k, sxm, int(w.stride(0)), sb,
-                               srm, srn, n, 1, None if part is None else part.data_ptr(), scratch_bytes, act,
-                               _raw_stream(dev))
+            s = sc if dense_sc else sc.contiguous()
+
+            def launch(y):
+                return call_wide(y.data_ptr(), x2.data_ptr(), w.data_ptr(), s.data_ptr(),
+                                 None if b is None else b.data_ptr(), bcode, None if r is None else r.data_ptr(), rcode,
+                                 m, n, k, sxm, int(w.stride(0)), sb, srm, srn, n, 1,
+                                 None if part is None else part.data_ptr(), scratch_bytes, act, _raw_stream(dev))
+
+            status = launch(y)
+            if status == FD_EUNSUPPORTED and o is not None:  # `out` may lie over an operand: write beside it
+                beside = x2.new_empty(expected)
+                status = launch(beside)
+                if status == 0:
+                    return o.copy_(beside)
             if status == FD_EUNSUPPORTED:
                 return slow(x2, w, sc, b, r, y, "the kernels' index range ends below these sizes")
             if status:

@@ -297,8 +297,9 @@ int fd_linear_fp8(void* y, const void* x, const void* w8, const float* w_scale,
  * with a call that may overlap); fd_linear_fp8_wide_scratch gives the bytes that
  * the preferred split needs (0: none). A smaller `scratch_bytes` lowers the
  * split, down to none with scratch NULL. The sums are added in a fixed order.
- * K % 16 == 0 and 16-byte aligned rows (else FD_EUNSUPPORTED). No reference
- * counterpart (see fd_linear_fp8).
+ * y may be row_add (the same elements in the same order) and must not overlap an
+ * operand otherwise. K % 16 == 0 and 16-byte aligned rows (either rule broken:
+ * FD_EUNSUPPORTED). No reference counterpart (see fd_linear_fp8).
  */
 int fd_linear_fp8_wide(void* y, const void* x, const void* w8, const float* w_scale,
                        const void* bias, int bias_dtype, const void* row_add, int row_dtype,
@@ -312,7 +313,7 @@ int fd_linear_fp8_wide_scratch(int64_t M, int64_t N, int64_t K, int64_t* bytes);
  * M > 16): mid[m,j] = round(silu(round(g)) * round(u)) with g and u the products
  * of x [M,H] (row stride sxm, already normalised) with rows j and I + j of
  * w_gate_up8 [2I,H] (contiguous), as fd_linear_fp8 computes them. mid is [M,I]
- * contiguous. H % 16 == 0 and 16-byte aligned rows (else FD_EUNSUPPORTED). No
+ * contiguous and overlaps none of the inputs. H % 16 == 0 and 16-byte aligned rows (else FD_EUNSUPPORTED). No
  * reference counterpart.
  */
 int fd_gate_up_fp8_wide(void* mid, const void* x, const void* w_gate_up8,

@@ -82,6 +82,28 @@ def test_scratch_lowers_the_split():
         check_product(y, x, q, s)
 
 
+@pytest.mark.parametrize("n,k", [(256, 2048), (256, 256), (40000, 64)])  # K splits, K = N, no split
+def test_output_over_an_operand(n, k):
+    """The output may hold row_add, a broadcast row of it, the bias or the activations: the product is whole first."""
+    import fused_decode as fd
+
+    m = 70
+    x, (q, s) = rnd(m, k, seed=20, dtype=torch.float16), fd.quantize_fp8(rnd(n, k, seed=21, scale=k**-0.5))
+    start = rnd(m, n, seed=22, dtype=torch.float16)
+    out, views = start.clone(), [lambda t: t, lambda t: t[:1], lambda t: t[-1], lambda t: t[:, :1], lambda t: t.flip(0)]
+    for view in views:
+        out.copy_(start)
+        assert fd.linear_decode_fp8(x, q, s, row_add=view(out), out=out) is out
+        assert torch.equal(out, fd.linear_decode_fp8(x, q, s, row_add=view(start)))
+    out.copy_(start)
+    fd.linear_decode_fp8(x, q, s, out[3], out=out)
+    assert torch.equal(out, fd.linear_decode_fp8(x, q, s, start[3]))
+    if n == k:
+        want, kept = fd.linear_decode_fp8(x, q, s, row_add=x), x.clone()
+        fd.linear_decode_fp8(x, q, s, row_add=x, out=x)
+        assert torch.equal(x, want) and not torch.equal(x, kept)
+
+
 def test_non_finite_values_stay_in_their_rows():
     """A NaN code reaches its output column, an infinite activation its row, nothing else."""
     import fused_decode as fd

@@ -60,6 +60,20 @@ def test_sizes_that_the_wide_kernels_refuse_are_still_computed(calls):
     assert torch.equal(y, product(x, q, s))
 
 
+def test_an_output_over_an_operand_is_written_beside_it(calls):
+    """The refused launch is made again on a fresh tensor, and `out` gets its values."""
+    x, q, s = fp8_case(m=20, n=64)
+    given = []
+
+    def wide(y, *args):
+        given.append(y)
+        return FD_EUNSUPPORTED if y == x.data_ptr() else FD_OK
+
+    calls.__dict__["linear_fp8_wide"] = wide
+    assert fp8.linear_decode_fp8(x, q, s, out=x) is x
+    assert len(given) == 2 and given[0] == x.data_ptr() != given[1]
+
+
 def test_an_mlp_whose_gate_up_is_refused_is_composed(calls):
     x, (gu, gs), (d, ds) = rnd(20, 64, seed=1, dtype=torch.bfloat16), *(fp8.quantize_fp8(rnd(*s, seed=i))
                                                                       for i, s in enumerate(((64, 64), (64, 32))))

@@ -44,6 +44,29 @@ def test_wide_sizes_end_below_the_index_range():
         assert refused(lib.fd_gate_up_fp8_wide(FAKE, FAKE, FAKE, FAKE, 32, 128, i, 128, 0, None))
 
 
+def test_wide_output_overlaps_no_operand():
+    """Tiles are stored while other workgroups read: only row_add, element for element, may be the output."""
+    from fused_decode import _lib as L
+
+    lib, m, n, k = L.lib(), 32, 64, 128
+    at = lambda i: 0x1000 + i * 0x100000
+    y, x, w, s, b, r = (at(i) for i in range(6))
+    over = lambda status: status == L.FD_EUNSUPPORTED and b"overlap" in lib.fd_last_error()
+
+    def lin(y=y, x=x, w=w, s=s, b=b, r=r, bdt=L.FD_F32, rdt=L.FD_F16, srm=n, srn=1):
+        return lib.fd_linear_fp8_wide(y, x, w, s, b, bdt, r, rdt, m, n, k, k, k, 1, srm, srn, n, 1, None, 0, L.FD_F16,
+                                      None)
+
+    last = m * n * 2 - 16  # bytes from the output's start to its last 16
+    for arg in ({"x": y}, {"x": y + last}, {"w": y + last}, {"s": y + last}, {"b": y}, {"r": y, "srm": 0},
+                {"r": y, "srm": 0, "srn": 0}, {"r": y + 16}, {"r": y, "srm": 1, "srn": m}, {"r": y, "rdt": L.FD_F32},
+                {"r": y, "rdt": L.FD_BF16}, {"y": x + (m * k - 1) * 2}, {"y": w + n * k - 16}, {"y": s + n * 4 - 16}):
+        assert over(lin(**arg)), arg
+    i = k
+    for arg in ((x, x, w, s), (w, x, w, s), (s, x, w, s), (x + (m * k - 8) * 2, x, w, s)):
+        assert lib.fd_gate_up_fp8_wide(*arg, m, k, i, k, 0, None) == L.FD_EINVAL
+
+
 def test_wide_scratch_follows_the_tiles():
     """No split, so no scratch, once the output tiles cover the GPU; else float32 sums for each split."""
     from fused_decode import _lib as L
