@@ -256,6 +256,11 @@ extern "C" int fd_linear_kn(void* y, const void* x, const void* w, const void* b
   if (N % 8 != 0 || !aligned16(w) || (K > 1 && swk % 8 != 0))
     return set_error(FD_EUNSUPPORTED, "the [K, N] GEMV needs N %% 8 == 0 and 16-byte aligned weight rows");
   if (N > 0x7fffffffLL - kKnCols || K > 0x7fffffffLL - 512) return set_error(FD_EUNSUPPORTED, "too large");
+  // one row of a column is written while the others' bias or broadcast row_add is still to be read
+  const int64_t ny = span_bytes(M, N, sym, syn, 2);
+  if ((bias && overlaps(y, ny, bias, span_bytes(1, N, 0, sb, dtype_bytes(bias_dtype)))) ||
+      row_add_meets(row_add, row_dtype, srm, srn, y, act_dtype, sym, syn, M, N))
+    return set_error(FD_EUNSUPPORTED, "y must not overlap bias, or row_add other than as row_add itself");
   int splits = kn_splits(M, N, K);
   if (!scratch) scratch_bytes = 0;
   while (splits > 1 && scratch_bytes < (int64_t)splits * M * N * 4) --splits;

@@ -262,8 +262,10 @@ int fd_pre_attn_qkv(void* y, void* normed, const void* hidden, const void* norm_
  * K is split over workgroups whose float32 sums go through `scratch`
  * (caller-owned, not shared with a call that may overlap); fd_linear_kn_scratch
  * gives the bytes of the preferred split (0: none). Less lowers the split, down
- * to none with scratch NULL. The sums are added in a fixed order. N % 8 == 0 and
- * 16-byte aligned rows of w (else FD_EUNSUPPORTED: fd_linear takes any strides).
+ * to none with scratch NULL. The sums are added in a fixed order. N % 8 == 0,
+ * 16-byte aligned rows of w, and a y that overlaps neither bias nor row_add other
+ * than as row_add itself, element for element (else FD_EUNSUPPORTED: fd_linear
+ * takes any strides and reads a column's operands before it writes the column).
  */
 int fd_linear_kn(void* y, const void* x, const void* w, const void* bias, int bias_dtype,
                  const void* row_add, int row_dtype, int64_t M, int64_t N, int64_t K, int64_t sxm,

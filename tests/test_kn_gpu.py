@@ -103,3 +103,21 @@ def test_kn_replays_from_a_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("m", [2, 16])
+@pytest.mark.parametrize("n,k", [(512, 1024), (70000, 64)])  # with K splits and without
+def test_kn_output_over_an_addend(m, n, k):
+    """The output may hold row_add, a broadcast row or column of it, or the bias."""
+    import fused_decode as fd
+
+    x, w = rnd(m, k, seed=13, dtype=torch.float16), rnd(k, n, seed=14, dtype=torch.float16, scale=k**-0.5).t()
+    start = rnd(m, n, seed=15, dtype=torch.float16)
+    out = start.clone()
+    for view in (lambda t: t, lambda t: t[:1], lambda t: t[-1]):
+        out.copy_(start)
+        assert fd.linear_decode(x, w, row_add=view(out), out=out) is out
+        check_product(out, x, w, view(start))
+    out.copy_(start)
+    fd.linear_decode(x, w, out[0], out=out)
+    check_product(out, x, w, start[0])

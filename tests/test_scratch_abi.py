@@ -98,3 +98,19 @@ def test_kn_entry_points_reject():
     assert lib.fd_linear_kn_scratch(4, 4096, 4096, ctypes.byref(out)) == L.FD_OK
     assert out.value > 0 and out.value % (4 * 4096 * 4) == 0
     assert lib.fd_linear_kn_scratch(4, 65536, 4096, ctypes.byref(out)) == L.FD_OK and out.value == 0
+
+
+def test_kn_output_overlaps_no_addend():
+    """A column's rows are written by several threads: a bias or a broadcast row_add in the output is refused."""
+    from fused_decode import _lib as L
+
+    lib, m, n, k = L.lib(), 4, 64, 128
+    y, x, w, b, r = (0x1000 + i * 0x100000 for i in range(5))
+
+    def lin(b=b, r=r, bdt=L.FD_F32, rdt=L.FD_F16, srm=n, srn=1):
+        return lib.fd_linear_kn(y, x, w, b, bdt, r, rdt, m, n, k, k, 1, n, 1, srm, srn, n, 1, None, 0, L.FD_F16, None)
+
+    last = m * n * 2 - 16
+    for arg in ({"b": y}, {"b": y + last}, {"r": y, "srm": 0}, {"r": y + last, "srm": 0}, {"r": y + 2},
+                {"r": y, "srm": 1, "srn": m}, {"r": y, "rdt": L.FD_F32}):
+        assert lin(**arg) == L.FD_EUNSUPPORTED and b"overlap" in lib.fd_last_error(), arg
