@@ -269,6 +269,15 @@ extern "C" int fd_add_rows(void* y, const void* a, const void* r, int r_dtype, c
     return set_error(FD_EUNSUPPORTED, "a and out need unit column stride");
   if (rows > kMaxPwWork || vectors > kMaxPwWork / rows || la->n > kMaxPwWork)
     return set_error(FD_EUNSUPPORTED, "tensor too large");
+  auto span = [](const fd_rows& l, int dt) {
+    return ((l.a - 1) * l.sa + (l.b - 1) * l.sb + (l.c - 1) * l.sc + (l.n - 1) * l.col + 1) * dtype_bytes(dt);
+  };
+  // r may be y element for element (a dim of one has no stride); any other overlap is read after it is written
+  auto same = [](int64_t dim, int64_t s, int64_t t) { return dim == 1 || s == t; };
+  if (overlaps(y, span(*ly, act_dtype), r, span(*lr, r_dtype)) &&
+      !(y == r && act_dtype == r_dtype && same(ly->a, ly->sa, lr->sa) && same(ly->b, ly->sb, lr->sb) &&
+        same(ly->c, ly->sc, lr->sc) && same(ly->n, ly->col, lr->col)))
+    return set_error(FD_EUNSUPPORTED, "y must not overlap r, other than as r itself");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint32_t tv = (uint32_t)(rows * vectors);
 #define FD_ADD_ROWS(T, R)                                                                                    \

@@ -482,22 +482,25 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
             add_rows, act, dev = native().add_rows, DTYPE_CODE[x.dtype], x.device.index
             r_rows, rcode = bytes(FdRows(1, 1, m, 0, 0, ra[0], ra[1], n)), DTYPE_CODE[row_add.dtype]
 
+        def add(dst, y, r):
+            return add_rows(dst.data_ptr(), y.data_ptr(), r.data_ptr(), rcode, dense, r_rows, dense, act,
+                            _raw_stream(dev))
+
         def fallback(x, w, b, r, out):
             x2, r2 = operands(x, r)
             y = F.linear(x2, w, b)
             if r2 is not None and y.dtype == x.dtype and y.is_contiguous() and _only_values(x, w, b, r):
                 if ra[2]:
                     r = r.expand(expected).reshape(m, n)
-                # straight into `out`, unless r might be part of it
-                direct = out is not None and out.untyped_storage().data_ptr() != r.untyped_storage().data_ptr()
-                status = add_rows((out if direct else y).data_ptr(), y.data_ptr(), r.data_ptr(), rcode, dense, r_rows,
-                                  dense, act, _raw_stream(dev))
+                # straight into `out`, unless r overlaps it
+                status = FD_EUNSUPPORTED if out is None else add(out, y, r)
                 if status == 0:
-                    if direct:
-                        return out
-                elif status == FD_EUNSUPPORTED:
+                    return out
+                if status == FD_EUNSUPPORTED:
+                    status = add(y, y, r)
+                if status == FD_EUNSUPPORTED:
                     y = (y.float() + r2.float()).to(x.dtype)
-                else:
+                elif status:
                     fail("fd_add_rows", status)
             elif r2 is not None:
                 y = (y.float() + r2.float()).to(x.dtype)

@@ -106,7 +106,8 @@ int fd_swiglu(void* y, const void* gate, const void* up, const fd_rows* lg,
  * y = round(a + r) in float32: the row_add of a product that is already in
  * memory (linear_decode above the GEMV's rows, kernels.py:657-672). a and y are
  * rows of unit column stride; r has any strides (0 = broadcast) and any of the
- * three dtypes. y may be a. Replaces no reference launcher (it adds in PyTorch,
+ * three dtypes. y may be a, or r element for element, and overlaps r in no other
+ * way (else FD_EUNSUPPORTED). Replaces no reference launcher (it adds in PyTorch,
  * ops.py:273-278).
  */
 int fd_add_rows(void* y, const void* a, const void* r, int r_dtype, const fd_rows* la,

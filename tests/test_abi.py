@@ -250,6 +250,22 @@ def _header_signatures() -> dict[str, str]:
     return sigs
 
 
+def test_add_rows_output_overlaps_no_addend(L):
+    """y may be r element for element; any other shared memory is read after it is written."""
+    lib, m, n = L.lib(), 20, 64
+    y, a, r = (0x1000 + i * 0x100000 for i in range(3))
+    grid = lambda row, col: ctypes.byref(L.FdRows(1, 1, m, 0, 0, row, col, n))
+
+    def add(r=r, rdt=L.FD_F16, row=n, col=1):
+        return lib.fd_add_rows(y, a, r, rdt, grid(n, 1), grid(row, col), grid(n, 1), L.FD_F16, None)
+
+    end = m * n * 2
+    for arg in ({"r": y, "row": 0}, {"r": y, "row": 0, "col": 0}, {"r": y + end - 2, "row": 0}, {"r": y + 2},
+                {"r": y, "row": 1, "col": m}, {"r": y, "rdt": L.FD_F32}, {"r": y, "rdt": L.FD_BF16},
+                {"r": y - end + 2}):
+        assert add(**arg) == L.FD_EUNSUPPORTED and b"overlap" in lib.fd_last_error(), arg
+
+
 def test_python_binding_matches_the_header():
     """fdcall.c converts each entry point's arguments by a code string: it must
     match the declaration in include/fused_decode.h argument for argument."""

@@ -74,6 +74,21 @@ def test_an_output_over_an_operand_is_written_beside_it(calls):
     assert len(given) == 2 and given[0] == x.data_ptr() != given[1]
 
 
+def test_a_row_add_over_the_output_is_added_before_it_is_copied(calls):
+    """The refused add into `out` is made again into the product, and `out` gets its values."""
+    x, w, out, given = rnd(20, 64, seed=1), rnd(32, 64, seed=2), rnd(20, 32, seed=3), []
+    x, w, out = (t.half() for t in (x, w, out))
+
+    def add_rows(y, *args):
+        given.append(y)
+        return FD_EUNSUPPORTED if y == out.data_ptr() else FD_OK
+
+    calls.__dict__["add_rows"] = add_rows
+    assert ops.linear_decode(x, w, row_add=out[:1], out=out) is out
+    assert len(given) == 2 and given[0] == out.data_ptr() != given[1]
+    assert torch.equal(out, torch.nn.functional.linear(x, w))  # the stand-in adds nothing
+
+
 def test_an_mlp_whose_gate_up_is_refused_is_composed(calls):
     x, (gu, gs), (d, ds) = rnd(20, 64, seed=1, dtype=torch.bfloat16), *(fp8.quantize_fp8(rnd(*s, seed=i))
                                                                       for i, s in enumerate(((64, 64), (64, 32))))

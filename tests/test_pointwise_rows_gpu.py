@@ -65,6 +65,19 @@ def test_row_add_that_is_part_of_the_output():
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("n", [64, 1001])
+def test_row_add_over_the_output(n):
+    """All of the output, a row or a column of it, and a row that comes by DLPack as a storage of its own."""
+    import fused_decode as fd
+
+    x, w, start = (rnd(*s, seed=i, dtype=torch.float16) for i, s in enumerate(((20, 48), (n, 48), (20, n))))
+    plain, out = F.linear(x, w).float(), start.clone()
+    for view in (lambda t: t, lambda t: t[-1], lambda t: t[:, :1], lambda t: torch.from_dlpack(t[7:8])):
+        out.copy_(start)
+        fd.linear_decode(x, w, row_add=view(out), out=out)
+        assert torch.equal(out, (plain + view(start).float()).half())
+
+
 def test_row_add_keeps_its_gradient():
     import fused_decode as fd
 
