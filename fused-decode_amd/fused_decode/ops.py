@@ -34,6 +34,7 @@ from typing import Callable, NamedTuple
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from ._checks import check
@@ -137,16 +138,27 @@ def _empty(shape, like: torch.Tensor) -> Callable[[torch.Tensor], torch.Tensor]:
     return lambda _ref: torch.empty(shape, dtype=dtype, device=device)
 
 
+def _watched() -> bool:
+    """Whether something records or replaces the torch calls made here, for which a launch on bare pointers would be
+    missing: tracing (torch.jit.trace, torch.compile), a dispatch mode (make_fx, fake tensors, counters) or a function
+    mode other than the default device's."""
+    if torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack():
+        return True
+    modes = torch._C._len_torch_function_stack()
+    return modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
+
+
 def _only_values(*tensors) -> bool:
     """Whether these are plain tensors that nothing records or transforms, so that a
     launch on their pointers says all that the torch formula would: no gradient
-    wanted, no forward-mode level, no vmap or tracing."""
-    if forward_ad._current_level >= 0 or torch.compiler.is_compiling():
+    wanted, no forward-mode level, no vmap, no tracing, no negation still to be made."""
+    if forward_ad._current_level >= 0 or _watched():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
         if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)
-                              or torch._C._functorch.is_functorch_wrapped_tensor(t)):
+                              or torch._C._functorch.is_functorch_wrapped_tensor(t)
+                              or torch._is_functional_tensor(t) or t.is_neg()):
             return False
     return True
 

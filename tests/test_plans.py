@@ -3,8 +3,13 @@ name and return a status, and the argument contract's device rule is left out.""
 
 from __future__ import annotations
 
+import warnings
+
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from fused_decode import fp8, ops
 from fused_decode._lib import FD_EUNSUPPORTED, FD_OK
@@ -48,6 +53,68 @@ def fp8_case(m=20, n=32, k=64):
 
 def product(x, q, s, row=0.0):
     return ((x.float() @ q.float().t()) * s + row).to(x.dtype)
+
+
+W, R = rnd(32, 64, seed=2).half(), rnd(20, 32, seed=3).half()
+Q, S = fp8.quantize_fp8(W)
+
+
+def wide_linear(x):
+    return ops.linear_decode(x, W, row_add=R)
+
+
+def wide_linear_fp8(x):
+    return fp8.linear_decode_fp8(x, Q, S, row_add=R)
+
+
+def formula(f, x):
+    if f is wide_linear:
+        return (torch.nn.functional.linear(x, W).float() + R.float()).half()
+    return product(x, Q, S, R.float())
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("f", [wide_linear, wide_linear_fp8])
+@pytest.mark.parametrize("trace", [make_fx, lambda f: lambda x: make_fx(f, pre_dispatch=True)(x),
+                                   lambda f: lambda x: torch.jit.trace(f, (x,), check_trace=False)])
+def test_a_traced_graph_holds_the_whole_product(calls, f, trace):
+    """Above the decode rows a graph traced on plain tensors computes the product, and row_add, of other inputs."""
+    x, other = rnd(20, 64, seed=1).half(), rnd(20, 64, seed=4).half()
+    graph = trace(f)(x)
+    assert calls == []
+    assert torch.equal(graph(other), formula(f, other))
+
+
+class Noting(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+class NotingFunctions(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("f", [wide_linear, wide_linear_fp8])
+def test_modes_see_the_products_torch_calls(calls, f):
+    x = rnd(20, 64, seed=1).half()
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", RuntimeWarning)
+        with Noting() as mode:
+            y = f(x)
+        assert calls == [] and any("add" in name or "mul" in name for name in mode.seen)
+        assert torch.equal(y, formula(f, x))
+        with NotingFunctions():
+            f(x)
+        assert calls == []
+    with torch.device("cpu"):  # the default device's function mode is no reason to leave the kernels
+        f(x)
+    assert calls == ["add_rows" if f is wide_linear else "linear_fp8_wide"]
 
 
 def test_sizes_that_the_wide_kernels_refuse_are_still_computed(calls):
