@@ -152,12 +152,12 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
         x2 = x.reshape(m, k)
         if x_copy:
             x2 = x2.contiguous()
+        if wide and not _only_values(x, w, sc, b, r):  # first: a transformed tensor has no pointer to ask for
+            return slow(x2, w, sc, b, r, y, "a gradient, a trace or a transform is asked for")
         if w.data_ptr() % 16:
             return slow(x2, w, sc, b, r, y, "the codes are not 16-byte rows with K % 16 == 0")
         if x2.data_ptr() % 16:
             return slow(x2, w, sc, b, r, y, "x rows are not 16-byte aligned with unit stride")
-        if wide and not _only_values(x, sc, b, r):
-            return slow(x2, w, sc, b, r, y, "a gradient or a transform is asked for")
         if r is not None and r_flat:  # indexed in place through (srm, srn), or copied when its dims do not merge
             r = r.expand(expected).reshape(m, n)
         if wide:
@@ -242,7 +242,7 @@ def _plan_mlp_fp8(hidden, norm_weight, w_gate_up, gate_up_scale, w_down, down_sc
 
         def wide(x, nw, wgu, sgu, wd, sd):
             normed = rms_norm(x, nw, eps=eps)
-            if wgu.data_ptr() % 16 or not _only_values(normed, sgu):
+            if not _only_values(normed, wgu, sgu) or wgu.data_ptr() % 16:
                 return products(x, normed, wgu, sgu, wd, sd)
             mid = normed.new_empty(mid_shape)
             status = gate_up(mid.data_ptr(), normed.data_ptr(), wgu.data_ptr(),

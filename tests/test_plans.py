@@ -7,6 +7,7 @@ import warnings
 
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.fx.experimental.proxy_tensor import make_fx
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -83,6 +84,34 @@ def test_a_traced_graph_holds_the_whole_product(calls, f, trace):
     graph = trace(f)(x)
     assert calls == []
     assert torch.equal(graph(other), formula(f, other))
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("f", [wide_linear, wide_linear_fp8])
+def test_functional_transforms_above_the_decode_rows(calls, f):
+    """Forward and reverse mode over the activations, and tensors without memory, take the torch formula."""
+    x, t = rnd(20, 64, seed=1).half(), rnd(20, 64, seed=4).half()
+    y, dy = torch.func.jvp(f, (x,), (t,))
+    assert torch.equal(y, formula(f, x))
+    weight = W.float() if f is wide_linear else Q.float() * S[:, None]
+    torch.testing.assert_close(dy.float(), t.float() @ weight.t(), rtol=1e-2, atol=1e-2)  # float16 roundings of it
+    y, vjp = torch.func.vjp(f, x)
+    (dx,) = vjp(torch.ones_like(y))
+    torch.testing.assert_close(dx.float(), weight.sum(0).expand(20, 64), rtol=1e-2, atol=1e-2)
+    assert torch.equal(torch.func.functionalize(f)(x), formula(f, x))
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        assert tuple(f(mode.from_tensor(x)).shape) == (20, 32)
+    assert calls == []
+
+
+@pytest.mark.filterwarnings("ignore")
+def test_gradients_of_the_scales_and_codes(calls):
+    """What eager autograd could differentiate above the decode rows, it still can: scales, and codes that ask for it."""
+    x, s, q = rnd(20, 64, seed=1).half(), S.clone().requires_grad_(), Q.clone().requires_grad_()
+    fp8.linear_decode_fp8(x, Q, s).sum().backward()
+    torch.testing.assert_close(s.grad, (x.float() @ Q.float().t()).sum(0))
+    assert fp8.linear_decode_fp8(x, q, S).requires_grad
+    assert calls == []
 
 
 class Noting(TorchDispatchMode):
