@@ -120,12 +120,12 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
     x2p = x.reshape(m, k)
     x_copy = x2p.stride(1) != 1  # gathered per call into contiguous rows
     why = None
-    if k == 0:
-        why = "K is 0" if m > _HAND_LIMIT else None
-    elif not (weight.stride(1) == 1 and (n == 1 or weight.stride(0) % 16 == 0) and k % 16 == 0):
+    if not (weight.stride(1) == 1 and (n == 1 or weight.stride(0) % 16 == 0) and k % 16 == 0):
         why = "the codes are not 16-byte rows with K % 16 == 0"
     elif not x_copy and m > 1 and x2p.stride(0) % 8 != 0:
         why = "x rows are not 16-byte aligned with unit stride"
+    elif k == 0 and m > _HAND_LIMIT:
+        why = "K is 0"
     if why is not None:
         if m > _HAND_LIMIT:
             why = f"{m} rows is above the decode kernels' {_HAND_LIMIT} and {why}"

@@ -156,6 +156,15 @@ def test_sizes_that_the_wide_kernels_refuse_are_still_computed(calls):
     assert torch.equal(y, product(x, q, s))
 
 
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("m", [1, 4, 16, 20])
+def test_no_k_leaves_the_bias_and_the_residual(calls, m):
+    """Empty E4M3 rows lie one element apart, which the kernels' 16-byte row rule refuses: computed by torch."""
+    x, q, b, r = torch.empty(m, 0).half(), torch.empty(8, 0).to(fp8.FP8_DTYPE), rnd(8, seed=1), rnd(m, 8, seed=2).half()
+    y = fp8.linear_decode_fp8(x, q, torch.ones(8), b, row_add=r)
+    assert calls == [] and torch.equal(y, (b + r.float()).half())
+
+
 def test_an_output_over_an_operand_is_written_beside_it(calls):
     """The refused launch is made again on a fresh tensor, and `out` gets its values."""
     x, q, s = fp8_case(m=20, n=64)
