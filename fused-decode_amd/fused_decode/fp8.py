@@ -13,7 +13,8 @@ activations, so the only approximation is the weight quantisation itself:
     y[m, n] = round(scale[n] * sum_k e4m3(q[n, k]) * x[m, k] + bias[n] + row_add[m, n])
 
 A decode GEMV at M <= 16 streams one byte per weight instead of two; above 16
-rows a tiled GEMM does, with the same arithmetic. There is no reference counterpart (the reference has fp16/bf16 weights only); this is the
+rows a tiled GEMM does, with the same arithmetic. There is no reference
+counterpart (the reference has fp16/bf16 weights only); this is the
 low-precision weight format its roadmap leaves for last.
 """
 
@@ -27,8 +28,8 @@ import torch
 from . import _lib
 from ._checks import check
 from ._lib import DTYPE_CODE, FD_EUNSUPPORTED, fail, native
-from .ops import (_FP8_ROWS, _PLANS, _check_out, _dense, _empty, _only_values, _plan_qkv, _raw_stream, _remember, _row_add_rows,
-                  _sig, rms_norm, swiglu)
+from .ops import (_FP8_ROWS, _PLANS, _check_out, _dense, _empty, _only_values, _plan_qkv, _raw_stream, _remember,
+                  _row_add_rows, _sig, _written, rms_norm, swiglu)
 
 FP8_MAX = 448.0
 FP8_DTYPE = torch.float8_e4m3fn
@@ -152,7 +153,7 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
         x2 = x.reshape(m, k)
         if x_copy:
             x2 = x2.contiguous()
-        if wide and not _only_values(x, w, sc, b, r):  # first: a transformed tensor has no pointer to ask for
+        if wide and not _only_values(x, w, sc, b, r, out=o):  # first: a transformed tensor has no pointer to ask for
             return slow(x2, w, sc, b, r, y, "a gradient, a trace or a transform is asked for")
         if w.data_ptr() % 16:
             return slow(x2, w, sc, b, r, y, "the codes are not 16-byte rows with K % 16 == 0")
@@ -180,7 +181,7 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
                 return slow(x2, w, sc, b, r, y, "the kernels' index range ends below these sizes")
             if status:
                 fail("fd_linear_fp8_wide", status)
-            return y
+            return y if o is None else _written(o)
         status = call(y.data_ptr(), x2.data_ptr(), w.data_ptr(), (sc if dense_sc else sc.contiguous()).data_ptr(),
                       None if b is None else b.data_ptr(), bcode, None if r is None else r.data_ptr(), rcode,
                       m, n, k, sxm, int(w.stride(0)), sb, srm, srn, n, 1, act, _raw_stream(dev))

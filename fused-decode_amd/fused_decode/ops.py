@@ -148,19 +148,31 @@ def _watched() -> bool:
     return modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
 
 
-def _only_values(*tensors) -> bool:
+def _only_values(*tensors, out: torch.Tensor | None = None) -> bool:
     """Whether these are plain tensors that nothing records or transforms, so that a
     launch on their pointers says all that the torch formula would: no gradient
-    wanted, no forward-mode level, no vmap, no tracing, no negation still to be made."""
+    wanted, no forward-mode level, no vmap, no tracing, no negation still to be made.
+    ``out``: the tensor that the launch writes, which torch would refuse to write in
+    place where it asks for a gradient or is an inference tensor outside that mode."""
     if forward_ad._current_level >= 0 or _watched():
         return False
+    if out is not None and out.is_inference() and not torch.is_inference_mode_enabled():
+        return False
     grad = torch.is_grad_enabled()
-    for t in tensors:
+    for t in (*tensors, out):
         if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)
                               or torch._C._functorch.is_functorch_wrapped_tensor(t)
                               or torch._is_functional_tensor(t) or t.is_neg()):
             return False
     return True
+
+
+def _written(out: torch.Tensor) -> torch.Tensor:
+    """``out`` after a launch wrote it, its version raised as an in-place torch call raises it, so that a backward
+    pass that saved its old values says so."""
+    if not out.is_inference():
+        torch.autograd.graph.increment_version(out)
+    return out
 
 
 # ------------------------------------------------------------------ norms
@@ -501,13 +513,13 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
         def fallback(x, w, b, r, out):
             x2, r2 = operands(x, r)
             y = F.linear(x2, w, b)
-            if r2 is not None and y.dtype == x.dtype and y.is_contiguous() and _only_values(x, w, b, r):
+            if r2 is not None and y.dtype == x.dtype and y.is_contiguous() and _only_values(x, w, b, r, out=out):
                 if ra[2]:
                     r = r.expand(expected).reshape(m, n)
                 # straight into `out`, unless r overlaps it
                 status = FD_EUNSUPPORTED if out is None else add(out, y, r)
                 if status == 0:
-                    return out
+                    return _written(out)
                 if status == FD_EUNSUPPORTED:
                     status = add(y, y, r)
                 if status == FD_EUNSUPPORTED:

@@ -114,6 +114,34 @@ def test_gradients_of_the_scales_and_codes(calls):
     assert calls == []
 
 
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("op", ["linear", "linear_fp8"])
+def test_outputs_that_torch_would_not_write_stay_refused(calls, op):
+    """A leaf that asks for its gradient, an inference tensor outside its mode; and a write raises the version."""
+    x, row = rnd(20, 64, seed=1).half(), R[0]
+
+    def run(out):
+        if op == "linear":
+            return ops.linear_decode(x, W, row_add=row, out=out)
+        return fp8.linear_decode_fp8(x, Q, S, row_add=row, out=out)
+
+    with pytest.raises(RuntimeError, match="leaf"):
+        run(torch.empty_like(R).requires_grad_())
+    with torch.inference_mode():
+        out = torch.empty_like(R)
+        assert run(out) is out
+    with pytest.raises(RuntimeError, match="inference"):
+        run(out)
+    a = torch.ones_like(R).requires_grad_()
+    out = torch.empty_like(R)
+    y = a * out
+    calls.clear()
+    run(out)
+    assert calls == ["add_rows" if op == "linear" else "linear_fp8_wide"]
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+
+
 class Noting(TorchDispatchMode):
     def __init__(self):
         super().__init__()
