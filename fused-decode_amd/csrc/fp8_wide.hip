@@ -47,16 +47,20 @@ enum WideEpi { WIDE_OUT = 0, WIDE_PART = 1, WIDE_SWIGLU = 2 };
 
 // One 16-byte-per-lane DMA into LDS at byte address `lds` (wave-uniform; lane L
 // lands at 16 L). The s_nop is the wait state a load that reads m0 needs after
-// the write of m0.
+// the write of m0. (m0 is a reserved register, which the compiler warns of; the clobber
+// still keeps it from reusing a value of its own across the asm.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <bool NT>
 __device__ __forceinline__ void wide_dma(const void* src, unsigned lds) {
   if constexpr (NT)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(src)
-                 : "memory");
+                 : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src)
-                 : "memory");
+                 : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // This wave's LDS reads have returned and its LDS writes are done, then the
 // workgroup's barrier; nothing moves across.

@@ -171,3 +171,17 @@ def test_quantize_fp8_on_cpu_matches_the_oracle():
     oq, os_ = O.fp8_quantize(w.numpy())
     assert q.dtype == torch.float8_e4m3fn and s.dtype == torch.float32
     assert np.array_equal(q.view(torch.uint8).numpy(), oq) and np.array_equal(s.numpy(), os_)
+
+
+def test_assembly_that_sets_m0_names_it():
+    """A kernel's inline assembly that writes m0 lists it as clobbered, so that no value of the compiler's is kept there."""
+    import re
+    from pathlib import Path
+
+    csrc, found = Path(__file__).resolve().parent.parent / "fused-decode_amd" / "csrc", 0
+    for src in sorted(csrc.glob("*.h*")):
+        for statement in re.findall(r"\basm\b(?: volatile)?\((.*?)\);", src.read_text(), re.S):
+            if re.search(r"\bs_\w+ m0,", statement):
+                found += 1
+                assert '"m0"' in statement, (src.name, statement)
+    assert found
