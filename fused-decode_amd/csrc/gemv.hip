@@ -1116,8 +1116,8 @@ int launch_mfma(int M, void* y, const void* x, const void* w, int N, int K, int6
   if (rp)
     return launch_dma_default<T, T, EPI_ROPE, false>(blocks, y, x, w, nullptr, M, N, K, sxm, swn, sym, syn,
                                                      e, r, nofold, st);
-  // a tile that names the default shape (linear_config's) leaves the rows open
-  const bool open = !t || ((t->waves == 0 || t->waves == 4) && (t->stages == 0 || t->stages == 2));
+  // a tile that names a shape has 16 rows; the default shape leaves the rows open
+  const bool open = !t || (t->waves == 0 && t->stages == 0);
   if (const int rows = open ? oct_rows(M, N, K, sizeof(T), e.ss != nullptr) : 0)
     return launch_oct<T, T>(rows, M, y, x, w, nullptr, N, K, sxm, swn, sym, syn, e, st);
 #define FD_DMA(NW, D)                                                                                        \

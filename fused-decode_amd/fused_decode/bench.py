@@ -875,6 +875,8 @@ def tune(dtype, out_path: str | None = None) -> dict:
                     br = 4 if m <= 4 else 8 if m <= 8 else 16
                     cands |= {(16, w, st) for w in (2, 4, 8) for st in (1, 2, 3)
                               if w * st * (256 + 16 * br) * 16 + w * 1024 <= 160 * 1024}
+                if dflt[0] == 16:  # what a launch that names no tile runs: rows left to the library
+                    dflt = (16, 0, 0)
                 cands.add(dflt)
                 times = {}
                 for t in sorted(cands):

@@ -196,6 +196,15 @@ def linear_config(kind: str, n: int, k: int, m: int | None = None) -> tuple[int,
     return rows, _BLOCK_K[kern], waves, stages
 
 
+def launch_tile(kind: str, n: int, k: int, m: int) -> tuple[int, int, int]:
+    """The (rows, waves, stages) that a launch names to the library: ``linear_config``'s, or for the MFMA GEMV where
+    neither the override nor the table names one, 16 rows with the rest left open, which lets the library take 8 or
+    24 rows where those load the CUs more evenly."""
+    rows, _, waves, stages = linear_config(kind, n, k, m)
+    named = os.environ.get("FUSED_DECODE_LINEAR") or tile_key(kind, n, k, m) in _tile_table()
+    return (rows, waves, stages) if named or rows != 16 else (16, 0, 0)
+
+
 def default_tile(kern: str, n: int, k: int) -> tuple[int, int, int]:
     """The library's own choice (rows, waves, stages) for a kernel ("simt" or "dot"):
     the MFMA GEMV runs four waves (two below four K units) with two units in
@@ -255,8 +264,7 @@ def linear_out(
         srm = 0 if row_add.shape[0] == 1 else int(row_add.stride(0))
         srn = 0 if row_add.shape[1] == 1 else int(row_add.stride(1))
     if tile is None:
-        rows, _, waves, stages = linear_config(kind, n, k, m)
-        tile = (rows, waves, stages)
+        tile = launch_tile(kind, n, k, m)
     status = native().linear_tiled(
         y.data_ptr(), x.data_ptr(), weight.data_ptr(), bias_ptr, bias_code, row_ptr, row_code,
         m, n, k, int(x.stride(0)), int(x.stride(1)), int(weight.stride(0)), int(weight.stride(1)),

@@ -42,7 +42,7 @@ from ._layout import contiguous_strides, plan_rows
 from ._lib import DTYPE_CODE, FD_EUNSUPPORTED, KIND_CODE, FdRows, FdTile, fail, native
 from .kernels import (
     _rms_env,
-    linear_config,
+    launch_tile,
     post_attn_mlp_out,
     pre_attn_qkv_out,
     resolve_kind,
@@ -461,7 +461,9 @@ def linear_decode(
     The HIP GEMV runs for a flattened batch up to ``DECODE_LINEAR_MAX_M`` rows
     (``SIMT_DECODE_LINEAR_MAX_M`` when FUSED_DECODE_LINEAR_KIND selects "simt"),
     or up to 16 when ``kind`` ("dot" or "simt") is given; wider batches call
-    ``F.linear`` (bit-identical to it), with row_add added in float32.
+    ``F.linear`` (bit-identical to it), with row_add added in float32. A weight
+    stored ``[K, N]`` (a transposed view) has kernels of its own, the same for
+    either kind.
     Reference: ops.py:212-280.
     """
     try:
@@ -534,8 +536,7 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
             return out
         return fallback
 
-    rows, _, waves, stages = linear_config(kind_r, n, k, m)
-    tile = bytes(FdTile(rows, waves, stages))
+    tile = bytes(FdTile(*launch_tile(kind_r, n, k, m)))
     call, act, kcode, dev = native().linear_tiled, DTYPE_CODE[x.dtype], KIND_CODE[kind_r], x.device.index
     swn, swk = int(weight.stride(0)), int(weight.stride(1))
     bcode = DTYPE_CODE[bias.dtype] if bias is not None else act

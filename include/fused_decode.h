@@ -149,8 +149,8 @@ int fd_linear(void* y, const void* x, const void* w, const void* bias, int bias_
  * keeps the activations in registers, whose waves then set how many 512-element
  * K chunks each lane holds). 0 = the library's default for that field; with rows
  * 0 the kernel is chosen as in fd_linear (MFMA for kind FD_KIND_DOT from M = 5).
- * The MFMA kernel in its default shape (waves 0 or 4, stages 0 or 2) takes 8 or 24
- * rows in place of 16 where those load the CUs more evenly.
+ * With waves and stages both 0 the MFMA kernel takes 8 or 24 rows in place of 16
+ * where those load the CUs more evenly; a tile that names either runs 16.
  */
 typedef struct fd_tile {
   int rows;

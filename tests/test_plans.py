@@ -3,6 +3,7 @@ name and return a status, and the argument contract's device rule is left out.""
 
 from __future__ import annotations
 
+import struct
 import warnings
 
 import pytest
@@ -12,7 +13,7 @@ from torch.fx.experimental.proxy_tensor import make_fx
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from fused_decode import fp8, ops
+from fused_decode import fp8, kernels, ops
 from fused_decode._lib import FD_EUNSUPPORTED, FD_OK
 
 
@@ -232,3 +233,24 @@ def test_an_mlp_whose_gate_up_is_refused_is_composed(calls):
     calls.status["gate_up_fp8_wide"] = FD_EUNSUPPORTED
     run()
     assert calls == ["rms_norm", "gate_up_fp8_wide", "linear_fp8_wide", "swiglu", "linear_fp8_wide"]
+
+
+def test_a_named_tile_runs_and_the_default_leaves_the_rows_open(calls, monkeypatch):
+    """Only a launch that names no shape (waves and stages 0) lets the library take 8 or 24 rows in place of 16."""
+    tiles = []
+    calls.__dict__["linear_tiled"] = lambda *args: tiles.append(struct.unpack("3i", args[19])) or FD_OK
+    monkeypatch.delenv("FUSED_DECODE_LINEAR", raising=False)
+    monkeypatch.delenv("FUSED_DECODE_LINEAR_KIND", raising=False)
+    monkeypatch.setattr(kernels, "_TILE_TABLE", {"dot:40x1024:m8": [16, 4, 2], "dot:40x1024:m9": [16, 2, 2]})
+    monkeypatch.setattr(kernels, "native", lambda: calls)
+    monkeypatch.setattr(kernels, "stream_of", lambda t: 0)
+    for n, m in ((32, 4), (32, 8), (32, 16), (40, 8), (40, 9)):
+        x, w = rnd(m, 1024, seed=m).half(), rnd(n, 1024, seed=n).half()
+        ops.linear_decode(x, w)
+        kernels.linear_out(x, w, torch.empty(m, n).half())
+        assert tiles[-1] == tiles[-2]
+    assert tiles[::2] == [(0, 2, 0), (16, 0, 0), (16, 0, 0), (16, 4, 2), (16, 2, 2)]
+    kernels.linear_out(x, w, torch.empty(m, n).half(), tile=(16, 4, 2))
+    monkeypatch.setenv("FUSED_DECODE_LINEAR", "16,128,4,2")
+    ops.linear_decode(x, w)
+    assert tiles[-2:] == [(16, 4, 2), (16, 4, 2)]
