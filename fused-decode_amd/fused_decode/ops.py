@@ -33,6 +33,7 @@ from typing import Callable, NamedTuple
 
 import torch
 import torch.nn.functional as F
+from torch import _C
 from torch.autograd import forward_ad
 from torch.utils._device import DeviceContext
 
@@ -139,31 +140,40 @@ def _empty(shape, like: torch.Tensor) -> Callable[[torch.Tensor], torch.Tensor]:
 
 
 def _watched() -> bool:
-    """Whether something records or replaces the torch calls made here, for which a launch on bare pointers would be
-    missing: tracing (torch.jit.trace, torch.compile), a dispatch mode (make_fx, fake tensors, counters) or a function
-    mode other than the default device's."""
-    if torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack():
+    """Whether something records, transforms or replaces the torch calls made here, for which a launch on bare pointers
+    would be missing: tracing (torch.jit.trace, torch.compile), forward mode, a torch.func transform, a dispatch mode
+    (make_fx, fake tensors, counters) or a function mode other than the default device's."""
+    if (forward_ad._current_level >= 0 or _C._functorch.peek_interpreter_stack() is not None or _C._is_tracing()
+            or _C._len_torch_dispatch_stack() or torch.compiler.is_compiling()):
         return True
-    modes = torch._C._len_torch_function_stack()
-    return modes > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
+    modes = _C._len_torch_function_stack()
+    return modes > 0 and any(type(_C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
 
 
 def _only_values(*tensors, out: torch.Tensor | None = None) -> bool:
-    """Whether these are plain tensors that nothing records or transforms, so that a
-    launch on their pointers says all that the torch formula would: no gradient
-    wanted, no forward-mode level, no vmap, no tracing, no negation still to be made.
-    ``out``: the tensor that the launch writes, which torch would refuse to write in
-    place where it asks for a gradient or is an inference tensor outside that mode."""
-    if forward_ad._current_level >= 0 or _watched():
+    """Whether nothing records or transforms these tensors (None: absent), so that a
+    launch on their pointers says all that the torch formula would: no subclass, no
+    gradient wanted, no negation still to be made, memory of their own (a tensor that
+    outlived its torch.func transform has none). ``out``: the tensor that the launch
+    writes, which torch would refuse to write in place where it asks for a gradient or
+    is an inference tensor outside that mode."""
+    if _watched():
         return False
-    if out is not None and out.is_inference() and not torch.is_inference_mode_enabled():
-        return False
-    grad = torch.is_grad_enabled()
-    for t in (*tensors, out):
-        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)
-                              or torch._C._functorch.is_functorch_wrapped_tensor(t)
-                              or torch._is_functional_tensor(t) or t.is_neg()):
+    if out is not None:
+        if out.is_inference() and not torch.is_inference_mode_enabled():
             return False
+        tensors += (out,)
+    grad = torch.is_grad_enabled()
+    try:
+        for t in tensors:
+            if t is not None:
+                kind = type(t)
+                if (kind is not torch.Tensor and kind is not torch.nn.Parameter) or (grad and t.requires_grad) \
+                        or t.is_neg():
+                    return False
+                t.data_ptr()
+    except RuntimeError:
+        return False
     return True
 
 

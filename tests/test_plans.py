@@ -100,8 +100,12 @@ def test_functional_transforms_above_the_decode_rows(calls, f):
     (dx,) = vjp(torch.ones_like(y))
     torch.testing.assert_close(dx.float(), weight.sum(0).expand(20, 64), rtol=1e-2, atol=1e-2)
     assert torch.equal(torch.func.functionalize(f)(x), formula(f, x))
+    kept = []
+    torch.func.vjp(lambda x: kept.append(x) or x, x)  # a wrapper that outlives its transform
+    assert torch.equal(f(kept[0]), formula(f, x))
     with FakeTensorMode(allow_non_fake_inputs=True) as mode:
         assert tuple(f(mode.from_tensor(x)).shape) == (20, 32)
+    assert torch.equal(f(torch._neg_view(-x)), formula(f, x))
     assert calls == []
 
 
