@@ -526,8 +526,7 @@ def _plan_linear(x, weight, bias, row_add, out, kind) -> Plan:
             x2, r2 = operands(x, r)
             y = F.linear(x2, w, b)
             if r2 is not None and y.dtype == x.dtype and y.is_contiguous() and _only_values(x, w, b, r, out=out):
-                if ra[2]:
-                    r = r.expand(expected).reshape(m, n)
+                r = r2 if ra[2] else r
                 # straight into `out`, unless r overlaps it
                 status = FD_EUNSUPPORTED if out is None else add(out, y, r)
                 if status == 0:

@@ -227,6 +227,15 @@ def test_a_row_add_over_the_output_is_added_before_it_is_copied(calls):
     assert torch.equal(out, torch.nn.functional.linear(x, w))  # the stand-in adds nothing
 
 
+def test_a_row_add_whose_dims_do_not_merge_is_gathered_once(calls):
+    x, r = rnd(2, 3, 4, 64, seed=1).half(), rnd(3, 2, 4, 32, seed=2).half().transpose(0, 1)
+    ops.linear_decode(x, W, row_add=r)
+    with torch.autograd.profiler.profile() as prof:
+        ops.linear_decode(x, W, row_add=r)
+    assert calls == ["add_rows"] * 2
+    assert [e.name for e in prof.function_events].count("aten::clone") == 1
+
+
 def test_an_mlp_whose_gate_up_is_refused_is_composed(calls):
     x, (gu, gs), (d, ds) = rnd(20, 64, seed=1, dtype=torch.bfloat16), *(fp8.quantize_fp8(rnd(*s, seed=i))
                                                                       for i, s in enumerate(((64, 64), (64, 32))))
