@@ -142,7 +142,7 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
     rcode = act if row_add is None else DTYPE_CODE[row_add.dtype]
     srm, srn, r_flat = ra if ra is not None else (0, 0, False)
     dense_sc = _dense(scale)
-    sxm = k if x_copy else int(x2p.stride(0))
+    sxm, swn = k if x_copy else int(x2p.stride(0)), int(weight.stride(0))
     call = native().linear_fp8
     wide = m > _HAND_LIMIT
     if wide:
@@ -155,26 +155,23 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
             x2 = x2.contiguous()
         if wide and not _only_values(x, w, sc, b, r, out=o):  # first: a transformed tensor has no pointer to ask for
             return slow(x2, w, sc, b, r, y, "a gradient, a trace or a transform is asked for")
-        if w.data_ptr() % 16:
+        xp, wp = x2.data_ptr(), w.data_ptr()
+        if wp % 16:
             return slow(x2, w, sc, b, r, y, "the codes are not 16-byte rows with K % 16 == 0")
-        if x2.data_ptr() % 16:
+        if xp % 16:
             return slow(x2, w, sc, b, r, y, "x rows are not 16-byte aligned with unit stride")
         if r is not None and r_flat:  # indexed in place through (srm, srn), or copied when its dims do not merge
             r = r.expand(expected).reshape(m, n)
         if wide:
             part = x2.new_empty(scratch_bytes // 4, dtype=torch.float32) if scratch_bytes else None
             s = sc if dense_sc else sc.contiguous()
-
-            def launch(y):
-                return call_wide(y.data_ptr(), x2.data_ptr(), w.data_ptr(), s.data_ptr(),
-                                 None if b is None else b.data_ptr(), bcode, None if r is None else r.data_ptr(), rcode,
-                                 m, n, k, sxm, int(w.stride(0)), sb, srm, srn, n, 1,
-                                 None if part is None else part.data_ptr(), scratch_bytes, act, _raw_stream(dev))
-
-            status = launch(y)
+            args = (xp, wp, s.data_ptr(), None if b is None else b.data_ptr(), bcode,
+                    None if r is None else r.data_ptr(), rcode, m, n, k, sxm, swn, sb, srm, srn, n, 1,
+                    None if part is None else part.data_ptr(), scratch_bytes, act, _raw_stream(dev))
+            status = call_wide(y.data_ptr(), *args)
             if status == FD_EUNSUPPORTED and o is not None:  # `out` may lie over an operand: write beside it
                 beside = x2.new_empty(expected)
-                status = launch(beside)
+                status = call_wide(beside.data_ptr(), *args)
                 if status == 0:
                     return o.copy_(beside)
             if status == FD_EUNSUPPORTED:
@@ -182,9 +179,9 @@ def _plan_linear_fp8(x, weight, scale, bias, row_add, out):
             if status:
                 fail("fd_linear_fp8_wide", status)
             return y if o is None else _written(o)
-        status = call(y.data_ptr(), x2.data_ptr(), w.data_ptr(), (sc if dense_sc else sc.contiguous()).data_ptr(),
+        status = call(y.data_ptr(), xp, wp, (sc if dense_sc else sc.contiguous()).data_ptr(),
                       None if b is None else b.data_ptr(), bcode, None if r is None else r.data_ptr(), rcode,
-                      m, n, k, sxm, int(w.stride(0)), sb, srm, srn, n, 1, act, _raw_stream(dev))
+                      m, n, k, sxm, swn, sb, srm, srn, n, 1, act, _raw_stream(dev))
         if status:
             fail("fd_linear_fp8", status)
         return y

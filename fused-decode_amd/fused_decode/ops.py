@@ -139,25 +139,26 @@ def _empty(shape, like: torch.Tensor) -> Callable[[torch.Tensor], torch.Tensor]:
     return lambda _ref: torch.empty(shape, dtype=dtype, device=device)
 
 
-def _watched() -> bool:
-    """Whether something records, transforms or replaces the torch calls made here, for which a launch on bare pointers
-    would be missing: tracing (torch.jit.trace, torch.compile), forward mode, a torch.func transform, a dispatch mode
-    (make_fx, fake tensors, counters) or a function mode other than the default device's."""
-    if (forward_ad._current_level >= 0 or _C._functorch.peek_interpreter_stack() is not None or _C._is_tracing()
-            or _C._len_torch_dispatch_stack() or torch.compiler.is_compiling()):
-        return True
-    modes = _C._len_torch_function_stack()
-    return modes > 0 and any(type(_C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
+# What a launch on bare pointers would be missing from: a torch.func transform, torch.jit.trace, a dispatch mode
+# (make_fx, fake tensors, counters), a function mode.
+_transform, _is_tracing = _C._functorch.peek_interpreter_stack, _C._is_tracing
+_dispatch_modes, _function_modes = _C._len_torch_dispatch_stack, _C._len_torch_function_stack
+
+
+def _function_modes_watch() -> bool:
+    """Whether a function mode other than the default device's is on."""
+    return any(type(_C._get_function_stack_at(i)) is not DeviceContext for i in range(_function_modes()))
 
 
 def _only_values(*tensors, out: torch.Tensor | None = None) -> bool:
-    """Whether nothing records or transforms these tensors (None: absent), so that a
-    launch on their pointers says all that the torch formula would: no subclass, no
-    gradient wanted, no negation still to be made, memory of their own (a tensor that
-    outlived its torch.func transform has none). ``out``: the tensor that the launch
-    writes, which torch would refuse to write in place where it asks for a gradient or
-    is an inference tensor outside that mode."""
-    if _watched():
+    """Whether nothing records or transforms a call on these tensors (None: absent), so
+    that a launch on their pointers says all that the torch formula would: no tracing,
+    transform or mode; no subclass, no gradient wanted, no negation still to be made,
+    memory of their own (a tensor that outlived its torch.func transform has none).
+    ``out``: the tensor that the launch writes, which torch would refuse to write in
+    place where it asks for a gradient or is an inference tensor outside that mode."""
+    if (torch.compiler.is_compiling() or forward_ad._current_level >= 0 or _transform() is not None or _is_tracing()
+            or _dispatch_modes() or (_function_modes() and _function_modes_watch())):
         return False
     if out is not None:
         if out.is_inference() and not torch.is_inference_mode_enabled():
@@ -180,8 +181,7 @@ def _only_values(*tensors, out: torch.Tensor | None = None) -> bool:
 def _written(out: torch.Tensor) -> torch.Tensor:
     """``out`` after a launch wrote it, its version raised as an in-place torch call raises it, so that a backward
     pass that saved its old values says so."""
-    if not out.is_inference():
-        torch.autograd.graph.increment_version(out)
+    torch.autograd.graph.increment_version(out)
     return out
 
 
