@@ -26,14 +26,16 @@
 // for lane group g, so a lane's 16 codes of one read feed both steps.
 //
 // What bounds it, at 120 bfloat16 rows and the widths of Llama-3-8B (H = 4096, I =
-// 14336): gate/up 39 us, of which its loads alone take 24 (117 MB of codes from
-// HBM and twice that in activations from L2, which a tile of all rows reads
-// once per 128 weight rows), its LDS reads, decodes and MFMAs alone 19, launch
-// and output 9; down 23 us and 6 for the sum over K splits. A layer's MLP 834 ->
-// 74 us against the float32 product of the decoded weights that these rows took
-// before (the weights written out in float32 and read again). The output first
-// left the kernel as 2-byte stores with the scales loaded per tile: 62 us for
-// gate/up.
+// 14336): gate/up 39 us (44 on another card, where the times below are longer alike),
+// of which its loads alone take 24 (117 MB of codes from HBM and twice that in
+// activations from L2, which a tile of all rows reads once per 128 weight rows),
+// its LDS reads, decodes and MFMAs alone 19, launch and output 9; down 23 us and 6
+// for the sum over K splits. No unit is full: matrix cores busy 29% of the cycles
+// (20% in down), LDS 13%, and the waves issue, wait to issue and wait for loads or
+// the barrier for a third of theirs each. A layer's MLP 834 -> 74 us against the
+// float32 product of the decoded weights that these rows took before (the weights
+// written out in float32 and read again). The output first left the kernel as 2-byte
+// stores with the scales loaded per tile: 62 us for gate/up.
 #include <type_traits>
 
 #include "fd_dma.h"
